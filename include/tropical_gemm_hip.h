@@ -191,6 +191,32 @@ size_t tg_gemm_noalloc_bytes(tg_semiring semiring, tg_dtype dtype, tg_layout lay
                              int64_t m, int64_t n, int64_t k);
 
 /*
+ * The (strided batched) product when its outputs are few or narrow, by a
+ * kernel of its own that needs no workspace and allocates nothing (fine under
+ * graph capture): tiles of 4 x 16 up to 32 x 32 outputs whose K is split over
+ * the lanes and waves of a workgroup.  *ran is 1 when the product was
+ * launched; 0 when another kernel is the faster one for these sizes (or they
+ * are empty): nothing was launched, and the caller goes on to one of the entry
+ * points below or above, which keep their own kernels (tg_gemm_plan).  The
+ * choice is made on dtype, sizes, strides and alignment.  Same arguments, values, argmax and
+ * errors as tg_gemm_strided_batched otherwise; batch 1 is the single product.
+ * No counterpart in the reference (one kernel per dtype).
+ */
+int tg_gemm_small(int device, tg_semiring semiring, tg_dtype dtype, tg_layout layout,
+                  const void* A, const void* B, void* C, int32_t* argmax, int64_t batch, int64_t m,
+                  int64_t n, int64_t k, int64_t stride_a, int64_t stride_b, int64_t stride_c,
+                  void* stream, int* ran);
+
+/* The launch tg_gemm_small would use ("16x16 waves 4": output tile and waves
+ * per workgroup), "none" when it would leave the problem to the other entry
+ * points, "invalid" for arguments the call would reject.  Strides 0 mean
+ * dense single products.  Host logic only, as tg_gemm_plan; diagnostic. */
+const char* tg_gemm_small_plan(tg_semiring semiring, tg_dtype dtype, tg_layout layout,
+                               const void* A, const void* B, const void* C, const int32_t* argmax,
+                               int64_t batch, int64_t m, int64_t n, int64_t k, int64_t stride_a,
+                               int64_t stride_b, int64_t stride_c);
+
+/*
  * Strided batched product: C[t] = A[t] (x) B[t] for t < batch, element
  * strides between consecutive matrices.  Replaces
  * launch_gemm_external_batched_with_argmax_f32 (kernels.rs:498-550, f32 only

@@ -23,6 +23,7 @@
 #include "tg_gemm_kresw.hpp"
 #include "tg_gemm_shortk.hpp"
 #include "tg_kernels.hpp"
+#include "tg_small.hpp"
 
 namespace {
 
@@ -1164,6 +1165,69 @@ int gemm_impl(int device, tg_semiring sr, tg_dtype dt, tg_layout layout, const v
     return rc;
 }
 
+tg::SmallProblem small_problem(tg_semiring sr, tg_dtype dt, const Problem& p) {
+    return tg::SmallProblem{int(sr), int(dt), p.A, p.B, p.C, p.IDX, p.batch, p.M, p.N, p.K,
+                            p.sA, p.sB, p.sC};
+}
+
+// Outputs (batch x M x N) below which the few-output kernel (tg_gemm_small.hpp)
+// is the faster one, by the path the problem would take otherwise.  Measured
+// on MI355X over 290 shapes of every dtype, with and without argmax (small /
+// other path, us; limits where the ratio nears 1):
+//   short K (<= 32): the other kernels are bound by the output writes, which
+//     leave in 1 KB runs there: f32 argmax 252 x 1672 x 18 8.6 / 8.7, 800 x
+//     672 x 16 9.7 / 7.5; value-only 800 x 672 x 16 5.4 / 6.8, 368 x 4848 x 16
+//     7.7 / 6.6.  Their 256-column tiles are mostly padding for narrow N:
+//     262144 x 16 x 16 argmax 29 / 114.
+//   direct-to-LDS and K-resident (32-bit, aligned): 900^3 f32 argmax 62 / 91,
+//     1024^3 84 / 59; i32 5376 x 64 x 64 9.6 / 9.5.
+//   generic tiles, 32-bit: 1001^3 f32 argmax 90 / 347, 872 x 4365 x 398 182 /
+//     393; value-only 243 x (48 x 262 x 420) 136 / 158.
+//   f64: 1024^3 argmax 203 / 271, value-only 143 / 202; argmax with K < 256 at
+//     100%..130% from half a million outputs (the exact mode there has
+//     no window loads).
+//   i64: 1024^3 argmax 198 / 260, 4 x (480 x 5084 x 428) 906 / 1093.
+int64_t small_output_limit(tg_dtype dt, const Plan& pl, const Problem& p) {
+    constexpr int64_t k1 = int64_t(1) << 10;
+    const bool argmax = p.IDX != nullptr;
+    const int64_t narrow = p.M < p.N ? p.M : p.N;
+    if (p.K <= 32) {
+        if (p.N <= 64) return INT64_MAX;
+        return !argmax ? 512 * k1 : dt == TG_F64 ? 128 * k1 : 256 * k1;
+    }
+    if (narrow <= 16) return INT64_MAX;  // tiles of the other kernels are mostly padding
+    switch (pl.path) {
+        case Path::SHORTK: return 512 * k1;
+        case Path::KRESW:
+        case Path::KRES8:
+        case Path::KRES: return dt == TG_I32 ? 256 * k1 : 512 * k1;
+        case Path::DL64:
+        case Path::DL64_VALUE: return 2048 * k1;
+        case Path::TILES_EXACT:
+        case Path::TILES_CHUNKED:
+        case Path::TILES: break;
+        default:  // direct-to-LDS, 32-bit
+            return narrow <= 32 ? 2048 * k1 : p.K >= 256 ? 896 * k1 : 512 * k1;
+    }
+    if (dt == TG_I64) return argmax ? 8192 * k1 : 4096 * k1;
+    if (dt == TG_F64) {
+        if (!argmax || pl.path == Path::TILES_CHUNKED) return 2048 * k1;
+        return p.K < 256 ? 512 * k1 : 1536 * k1;
+    }
+    return !argmax || p.K <= 96 ? 2048 * k1 : 4096 * k1;
+}
+
+// True when tg_gemm_small takes the problem: `form` is its launch.
+bool choose_small(tg_semiring sr, tg_dtype dt, const Problem& p, tg::SmallForm* form) {
+    if (p.batch <= 0 || p.M <= 0 || p.N <= 0 || p.K <= 0) return false;
+    const Plan pl = plan_gemm(sr, dt, p, workspace_bytes_for(dt, p.batch, p.M, p.N, p.K,
+                                                             p.IDX != nullptr));
+    // In floating point: batch * M * N of a caller's sizes may pass 2^63.
+    if (double(p.batch) * double(p.M) * double(p.N) >= double(small_output_limit(dt, pl, p)))
+        return false;
+    return tg::small_form(small_problem(sr, dt, p), form);
+}
+
 // ----------------------------------------------------------------------------
 // Workspace without allocation (tg_gemm_noalloc)
 // ----------------------------------------------------------------------------
@@ -1619,6 +1683,46 @@ int tg_gemm(int device, tg_semiring semiring, tg_dtype dtype, tg_layout layout, 
             void* stream) {
     return gemm_impl(device, semiring, dtype, layout, A, B, C, argmax, 1, m, n, k, 0, 0, 0, false,
                      nullptr, 0, false, stream);
+}
+
+int tg_gemm_small(int device, tg_semiring semiring, tg_dtype dtype, tg_layout layout,
+                  const void* A, const void* B, void* C, int32_t* argmax, int64_t batch, int64_t m,
+                  int64_t n, int64_t k, int64_t stride_a, int64_t stride_b, int64_t stride_c,
+                  void* stream, int* ran) {
+    if (ran == nullptr) return fail(TG_ERR_INVALID_ARGUMENT, "ran is NULL");
+    *ran = 0;
+    int rc = validate_forward(semiring, dtype, layout, A, B, C, batch, m, n, k, stride_a, stride_b,
+                              stride_c, true);
+    if (rc != TG_OK) return rc;
+    const Problem p = make_problem(layout, A, B, C, argmax, batch, m, n, k, stride_a, stride_b,
+                                   stride_c, true);
+    tg::SmallForm form;
+    if (!choose_small(semiring, dtype, p, &form)) return TG_OK;
+    rc = select_device(device);
+    if (rc != TG_OK) return rc;
+    hipStream_t st = as_stream(stream);
+    KernelTimer timer(st);
+    TG_HIP(tg::small_launch(small_problem(semiring, dtype, p), form, st));
+    *ran = 1;
+    return TG_OK;
+}
+
+const char* tg_gemm_small_plan(tg_semiring semiring, tg_dtype dtype, tg_layout layout,
+                               const void* A, const void* B, const void* C, const int32_t* argmax,
+                               int64_t batch, int64_t m, int64_t n, int64_t k, int64_t stride_a,
+                               int64_t stride_b, int64_t stride_c) {
+    static thread_local std::string name;
+    const bool strided = stride_a != 0 || stride_b != 0 || stride_c != 0;
+    if (validate_forward(semiring, dtype, layout, A, B, C, batch, m, n, k, stride_a, stride_b,
+                         stride_c, strided) != TG_OK)
+        return "invalid";
+    const Problem p = make_problem(layout, A, B, const_cast<void*>(C), const_cast<int32_t*>(argmax),
+                                   batch, m, n, k, stride_a, stride_b, stride_c, strided);
+    tg::SmallForm f;
+    if (!choose_small(semiring, dtype, p, &f)) return "none";
+    name = std::to_string(4 * f.lr) + "x" + std::to_string(4 * f.lc) + " waves " +
+           std::to_string(f.waves);
+    return name.c_str();
 }
 
 int tg_gemm_noalloc(int device, tg_semiring semiring, tg_dtype dtype, tg_layout layout,

@@ -684,7 +684,7 @@ __global__ __launch_bounds__(256) void tg_transpose_v(const T* __restrict__ B, T
 // Zero fill (16-byte stores + byte tail).  Used instead of hipMemsetAsync so
 // that the library records no memset nodes when a caller captures a graph.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void tg_fill_zero(unsigned char* __restrict__ p, int64_t bytes) {
+static __global__ __launch_bounds__(256) void tg_fill_zero(unsigned char* __restrict__ p, int64_t bytes) {
     const int64_t nvec = bytes / 16;
     const int64_t stride = int64_t(gridDim.x) * 256;
     for (int64_t v = int64_t(blockIdx.x) * 256 + threadIdx.x; v < nvec; v += stride)

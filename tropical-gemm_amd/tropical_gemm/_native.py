@@ -55,6 +55,10 @@ SIGNATURES = {
     "tg_gemm": ([_i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp], _i32),
     "tg_gemm_noalloc": ([_i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp], _i32),
     "tg_gemm_noalloc_bytes": ([_i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i64], _sz),
+    "tg_gemm_small": ([_i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
+                       _i64, _i64, _vp, ctypes.POINTER(_i32)], _i32),
+    "tg_gemm_small_plan": ([_i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
+                            _i64, _i64], ctypes.c_char_p),
     "tg_gemm_workspace_size": ([_i32, _i64, _i64, _i64, _i64, _i32], _sz),
     "tg_gemm_ws": ([_i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _sz, _vp],
                    _i32),
@@ -140,6 +144,17 @@ def gemm_plan(semiring: str, dtype: str, m: int, n: int, k: int, with_argmax: bo
     return lib.tg_gemm_plan(SEMIRING[semiring], DTYPE[dtype], LAYOUT[layout], a, b, c,
                             i if with_argmax else None, batch, m, n, k, *strides,
                             workspace_bytes).decode()
+
+
+def gemm_small_plan(semiring: str, dtype: str, m: int, n: int, k: int, with_argmax: bool = True,
+                    layout: str = "row", batch: int = 1, strides=(0, 0, 0),
+                    addresses=(256, 256, 256, 256)) -> str:
+    """The launch the few-output kernel would use for a product, or "none"
+    (host logic only)."""
+    a, b, c, i = addresses
+    return load().tg_gemm_small_plan(SEMIRING[semiring], DTYPE[dtype], LAYOUT[layout], a, b, c,
+                                     i if with_argmax else None, batch, m, n, k,
+                                     *strides).decode()
 
 
 def last_error() -> str:

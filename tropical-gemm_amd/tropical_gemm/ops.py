@@ -57,6 +57,26 @@ def _check_pair(a: torch.Tensor, b: torch.Tensor, ndim: int) -> None:
                          f"(got {a.device.type}); move the tensors to the GPU first")
 
 
+def _product(semiring: str, a, b, c, am, batch: int, m: int, n: int, k: int) -> None:
+    """C (and argmax) of contiguous row-major operands: the few-output kernel
+    where it is the faster one (no workspace), tg_gemm_strided_batched_ws
+    otherwise."""
+    lib = nat.load()
+    dev = a.device
+    dt = nat.DTYPE[_DT[a.dtype]]
+    args = (dev.index or 0, nat.SEMIRING[semiring], dt, nat.LAYOUT["row"], a.data_ptr(),
+            b.data_ptr(), c.data_ptr(), None if am is None else am.data_ptr(), batch, m, n, k,
+            m * k, k * n, m * n)
+    stream = torch.cuda.current_stream(dev).cuda_stream
+    ran = ctypes.c_int(0)
+    nat.check(lib.tg_gemm_small(*args, stream, ran))
+    if ran.value:
+        return
+    ws_bytes = lib.tg_gemm_workspace_size(dt, batch, m, n, k, 0 if am is None else 1)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+    nat.check(lib.tg_gemm_strided_batched_ws(*args, _ptr(ws), ws_bytes, stream))
+
+
 def gemm(semiring: str, a, b, with_argmax: bool = True):
     """Row-major ``C = A (x) B`` on the GPU.  Returns ``(C, argmax)`` with
     ``argmax`` int32 (``None`` when ``with_argmax`` is False)."""
@@ -72,13 +92,7 @@ def gemm(semiring: str, a, b, with_argmax: bool = True):
     dev = a.device
     c = torch.empty((m, n), dtype=a.dtype, device=dev)
     am = torch.empty((m, n), dtype=torch.int32, device=dev) if with_argmax else None
-    lib = nat.load()
-    dt = nat.DTYPE[_DT[a.dtype]]
-    ws_bytes = lib.tg_gemm_workspace_size(dt, 1, m, n, k, 1 if with_argmax else 0)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-    nat.check(lib.tg_gemm_ws(dev.index or 0, nat.SEMIRING[semiring], dt, nat.LAYOUT["row"],
-                             _ptr(a), _ptr(b), _ptr(c), _ptr(am), m, n, k, _ptr(ws), ws_bytes,
-                             _stream(dev)))
+    _product(semiring, a, b, c, am, 1, m, n, k)
     return c, am
 
 
@@ -98,13 +112,7 @@ def gemm_batched(semiring: str, a, b, with_argmax: bool = True):
     dev = a.device
     c = torch.empty((batch, m, n), dtype=a.dtype, device=dev)
     am = torch.empty((batch, m, n), dtype=torch.int32, device=dev) if with_argmax else None
-    lib = nat.load()
-    dt = nat.DTYPE[_DT[a.dtype]]
-    ws_bytes = lib.tg_gemm_workspace_size(dt, batch, m, n, k, 1 if with_argmax else 0)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-    nat.check(lib.tg_gemm_strided_batched_ws(
-        dev.index or 0, nat.SEMIRING[semiring], dt, nat.LAYOUT["row"], _ptr(a), _ptr(b), _ptr(c),
-        _ptr(am), batch, m, n, k, m * k, k * n, m * n, _ptr(ws), ws_bytes, _stream(dev)))
+    _product(semiring, a, b, c, am, batch, m, n, k)
     return c, am
 
 
