@@ -502,6 +502,42 @@ int run_gemm_dl(const Problem& p, void* ws, int splits, hipStream_t st) {
     return TG_OK;
 }
 
+// Direct-to-LDS kernel with element loads (32-bit types; N, K, strides and
+// pointers of any alignment), 64 x 64 tiles, unsplit.  With argmax the
+// workspace holds B^T.
+template <int SR, typename T, bool ARGMAX, int CL>
+int run_gemm_dl_elem(const Problem& p, void* ws, hipStream_t st) {
+    using Cfg = tg::DlCfg<4, 4>;
+    const int64_t tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM;
+    const int64_t tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
+    if (tiles_m * tiles_n > 0x7fffffffLL)
+        return fail(TG_ERR_DIMENSION_MISMATCH, "output too large for one launch");
+    if (ARGMAX && (p.K + 31) / 32 > 65535)
+        return fail(TG_ERR_DIMENSION_MISMATCH, "K too large for the transpose grid");
+    T* const BT = ARGMAX ? static_cast<T*>(ws) : nullptr;
+    const int64_t sBT = p.K * p.N;
+    const T* A = static_cast<const T*>(p.A);
+    const T* B = static_cast<const T*>(p.B);
+    T* C = static_cast<T*>(p.C);
+    for (int64_t z0 = 0; ARGMAX && z0 < p.batch; z0 += 65535) {
+        const int64_t nb = (p.batch - z0 < 65535) ? p.batch - z0 : 65535;
+        const int rc = launch_transpose<T>(B + z0 * p.sB, BT + z0 * sBT, p.K, p.N, p.sB, sBT, nb, st);
+        if (rc != TG_OK) return rc;
+    }
+    KernelTimer timer(st);
+    for (int64_t z0 = 0; z0 < p.batch; z0 += 65535) {
+        const int64_t nb = (p.batch - z0 < 65535) ? p.batch - z0 : 65535;
+        dim3 grid(unsigned(tiles_m * tiles_n), 1, unsigned(nb));
+        hipLaunchKernelGGL((tg::tg_gemm_dl<SR, T, ARGMAX, 4, 4, CL, true, false, 0, 1, true>), grid,
+                           dim3(256), ARGMAX ? Cfg::LDS_BYTES : Cfg::TILE_BYTES, st, A + z0 * p.sA,
+                           B + z0 * p.sB, ARGMAX ? BT + z0 * sBT : nullptr, C + z0 * p.sC,
+                           ARGMAX ? p.IDX + z0 * p.sC : nullptr, p.M, p.N, p.K, p.sA, p.sB, p.sC,
+                           int(tiles_m), int(tiles_n), p.K, int64_t(0));
+        TG_HIP(hipGetLastError());
+    }
+    return TG_OK;
+}
+
 // Compute units of the current device (cached per device).
 int current_cu_count() {
     static std::mutex mu;
@@ -718,7 +754,7 @@ constexpr int64_t kShortkArgmaxMaxK = 32;
 constexpr int64_t kShortkValueMaxK = 63;
 
 // The kernel a problem runs on.
-enum class Path { SHORTK, KRESW, KRES8, KRES, DL_88_32, DL_48_16, DL_48_VALUE, DL_44_8, DL_44_16, DL_44_32, DL64, DL64_VALUE, TILES_EXACT, TILES_CHUNKED, TILES };
+enum class Path { SHORTK, KRESW, KRES8, KRES, DL_88_32, DL_48_16, DL_48_VALUE, DL_44_8, DL_44_16, DL_44_32, DL_ELEM_8, DL_ELEM_16, DL_ELEM, DL64, DL64_VALUE, TILES_EXACT, TILES_CHUNKED, TILES };
 
 struct Plan {
     Path path = Path::TILES;
@@ -733,6 +769,7 @@ bool uses_workspace(const Plan& pl, bool argmax) {
         case Path::KRESW:
         case Path::KRES8:
         case Path::KRES:
+        case Path::DL_ELEM:
         case Path::TILES_EXACT:
         case Path::TILES: return false;
         case Path::TILES_CHUNKED:
@@ -853,6 +890,27 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
             }
             pl.splits = 1;
         }
+        // Rows or operands that are not whole 16-byte vectors: the
+        // direct-to-LDS kernel with element loads, from a quarter of the
+        // CUs' worth of tiles up.  Measured on MI355X against the generic
+        // kernel (us): argmax 2001^3 f32 348 / 750, i32 455 / 807, 701^3 75 /
+        // 301, 3001 x 1501 x 301 102 / 182, 3001^2 x 100 104 / 121, x 65
+        // 91 / 86 (so up to K = 96 the exact mode stays); value-only 2001^3
+        // 291 / 342, 2001^2 x 60 15.5 / 22.8.  Below K = 48 most of a second
+        // k-tile would be padding.
+        const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
+        if (tiles64 >= 64 && tg::dl_elem_fits<8>(p.M, p.N, p.K)) {
+            if (!argmax && p.K >= 48) {
+                pl.path = Path::DL_ELEM;
+                return pl;
+            }
+            const tg_dtype dt = std::is_same<T, float>::value ? TG_F32 : TG_I32;
+            if (argmax && p.K > kExactPartialMaxK &&
+                ws_layout(dt, p.batch, p.M, p.N, p.K, true, 1).total <= ws_bytes) {
+                pl.path = p.K <= 512 ? Path::DL_ELEM_8 : Path::DL_ELEM_16;
+                return pl;
+            }
+        }
     }
     if constexpr (std::is_same<T, double>::value) {
         // f64 on at least 256 tiles of 64 x 128 with the workspace for the
@@ -902,6 +960,9 @@ int run_gemm_typed(const Problem& p, void* ws, size_t ws_bytes, hipStream_t st) 
             case Path::DL_44_8: return run_gemm_dl<SR, T, 4, 4, 8>(p, ws, pl.splits, st);
             case Path::DL_44_16: return run_gemm_dl<SR, T, 4, 4, 16>(p, ws, pl.splits, st);
             case Path::DL_44_32: return run_gemm_dl<SR, T, 4, 4, 32>(p, ws, pl.splits, st);
+            case Path::DL_ELEM_8: return run_gemm_dl_elem<SR, T, true, 8>(p, ws, st);
+            case Path::DL_ELEM_16: return run_gemm_dl_elem<SR, T, true, 16>(p, ws, st);
+            case Path::DL_ELEM: return run_gemm_dl_elem<SR, T, false, 32>(p, ws, st);
             default: break;
         }
     }
@@ -1019,6 +1080,9 @@ const char* path_name(Path path) {
         case Path::DL_44_8: return "dl_4x4_cl8";
         case Path::DL_44_16: return "dl_4x4_cl16";
         case Path::DL_44_32: return "dl_4x4_cl32";
+        case Path::DL_ELEM_8: return "dl_elem_cl8";
+        case Path::DL_ELEM_16: return "dl_elem_cl16";
+        case Path::DL_ELEM: return "dl_elem";
         case Path::DL64: return "dl64_4x8_cl16";
         case Path::DL64_VALUE: return "dl64_4x8";
         case Path::TILES_EXACT: return "tiles_exact";
@@ -1150,8 +1214,19 @@ int gemm_impl(int device, tg_semiring sr, tg_dtype dt, tg_layout layout, const v
     if (!ws_given) {
         // Allocate the full workspace only for the kernels that read it.
         ws_bytes = workspace_bytes_for(dt, batch, m, n, k, with_argmax);
-        if (ws_bytes > 0 && !uses_workspace(plan_gemm(sr, dt, p, ws_bytes), with_argmax))
-            ws_bytes = 0;
+        if (ws_bytes > 0) {
+            const Plan pl = plan_gemm(sr, dt, p, ws_bytes);
+            if (!uses_workspace(pl, with_argmax)) {
+                ws_bytes = 0;
+            } else if (pl.path == Path::DL_ELEM_8 &&
+                       !uses_workspace(plan_gemm(sr, dt, p, 0), with_argmax)) {
+                // Under capture a product that can do without a workspace
+                // stays free of allocation nodes.
+                hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+                if (hipStreamIsCapturing(st, &cap) != hipSuccess) (void)hipGetLastError();
+                if (cap != hipStreamCaptureStatusNone) ws_bytes = 0;
+            }
+        }
         if (ws_bytes > 0) {
             TG_HIP(hipMallocAsync(&work, ws_bytes, st));
             own = true;
@@ -1181,8 +1256,10 @@ tg::SmallProblem small_problem(tg_semiring sr, tg_dtype dt, const Problem& p) {
 //     262144 x 16 x 16 argmax 29 / 114.
 //   direct-to-LDS and K-resident (32-bit, aligned): 900^3 f32 argmax 62 / 91,
 //     1024^3 84 / 59; i32 5376 x 64 x 64 9.6 / 9.5.
-//   generic tiles, 32-bit: 1001^3 f32 argmax 90 / 347, 872 x 4365 x 398 182 /
-//     393; value-only 243 x (48 x 262 x 420) 136 / 158.
+//   direct-to-LDS with element loads (32-bit, unaligned): argmax 1531 x 777 x
+//     999 f32 104 / 114, 7 x (500 x 501 x 502) 88 / 74; value-only 81 / 87, 57 / 44.
+//   generic tiles, 32-bit (few tiles, or K <= 96): 42 x (452 x 92 x 52) f32
+//     argmax 23 / 28, 2001^2 x 60 45 / 41.
 //   f64: 1024^3 argmax 203 / 271, value-only 143 / 202; argmax with K < 256 at
 //     100%..130% from half a million outputs (the exact mode there has
 //     no window loads).
@@ -1206,6 +1283,10 @@ int64_t small_output_limit(tg_dtype dt, const Plan& pl, const Problem& p) {
         case Path::TILES_EXACT:
         case Path::TILES_CHUNKED:
         case Path::TILES: break;
+        case Path::DL_ELEM_8:
+        case Path::DL_ELEM_16:
+        case Path::DL_ELEM:
+            return narrow <= 32 || (argmax && p.K < 256) ? 2048 * k1 : 1280 * k1;
         default:  // direct-to-LDS, 32-bit
             return narrow <= 32 ? 2048 * k1 : p.K >= 256 ? 896 * k1 : 512 * k1;
     }
@@ -1214,7 +1295,7 @@ int64_t small_output_limit(tg_dtype dt, const Plan& pl, const Problem& p) {
         if (!argmax || pl.path == Path::TILES_CHUNKED) return 2048 * k1;
         return p.K < 256 ? 512 * k1 : 1536 * k1;
     }
-    return !argmax || p.K <= 96 ? 2048 * k1 : 4096 * k1;
+    return 2048 * k1;
 }
 
 // True when tg_gemm_small takes the problem: `form` is its launch.

@@ -93,6 +93,12 @@ __device__ __forceinline__ void lds_load16(const void* src, void* dst) {
     __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
 }
 
+// The same with one 4-byte element per lane: LDS at dst + lane * 4, so src
+// needs the alignment of an element only.
+__device__ __forceinline__ void lds_load4(const void* src, void* dst) {
+    __builtin_amdgcn_global_load_lds(src, dst, 4, 0, 0);
+}
+
 // Byte address of a pointer into LDS, as ds_* instructions take it (the low
 // 32 bits of the generic address are the offset in the LDS aperture).
 __device__ __forceinline__ uint32_t lds_byte_addr(const void* p) {
@@ -172,6 +178,16 @@ inline bool dl_fits(int64_t M, int64_t N, int64_t K, int64_t sA, int64_t sB, int
 // fit 32 bits.
 inline bool pipe_fits(int64_t N, int64_t K) {
     return K < (int64_t(1) << 23) && N < (int64_t(1) << 25);
+}
+
+// True when the element-load instantiation (ELEM) of tg_gemm_dl<.., CL> can
+// run the problem: any alignment, N and K (from 4: a resolve window's quad
+// that would pass the end of a row shifts back into it); 32-bit lane offsets
+// inside a tile's 64 rows of A and one row of B, 16-bit chunk slots.
+template <int CL>
+inline bool dl_elem_fits(int64_t M, int64_t N, int64_t K) {
+    return M > 0 && N > 0 && K >= 4 && (K + CL - 1) / CL < 0xFFFF && K < (int64_t(1) << 24) &&
+           N < (int64_t(1) << 28);
 }
 
 // True when every tile of the problem is full.
@@ -303,8 +319,14 @@ __device__ __forceinline__ void record4(int32_t& c0, int32_t& c1, int32_t& c2, i
 // read from LDS while the current pair is folded (reads issued ahead and
 // waited for explicitly), so a wave does not stall on LDS between pairs
 // (MaxPlus f32 4096^3 on MI355X: 1.847 against 1.891 ms).
+// ELEM (with TAILK; any K): the tiles are loaded one element per lane, so N,
+// K, the batch strides and the pointers need no 16-byte alignment: four times
+// the load instructions (16 instead of 4 per wave and 64 x 64 k-tile, against
+// ~900 others), the same LDS layout.  MaxPlus f32 2048^3 on MI355X: argmax 402
+// us against 375 with 16-byte loads (11 us of it the element transpose),
+// value-only 290.
 template <int SR, typename T, bool ARGMAX, int TM_, int TN_, int CL, bool TAILK = false,
-          bool BDIRECT = false, int PIPE = 0, int HALVES = 1>
+          bool BDIRECT = false, int PIPE = 0, int HALVES = 1, bool ELEM = false>
 __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_per_eu(
     PIPE != 0 ? PIPE : ARGMAX ? DlCfg<TM_, TN_>::WAVES_ARGMAX : DlCfg<TM_, TN_>::WAVES_VALUE))) void tg_gemm_dl(
     const T* __restrict__ A, const T* __restrict__ B, const T* __restrict__ BT,
@@ -319,6 +341,7 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
     static_assert(!ARGMAX || TM == 4, "argmax tiles have 4 rows per thread");
     static_assert(HALVES == 1 || ((HALVES == 2 || HALVES == 4) && ARGMAX && !TAILK && PIPE == 0),
                   "K slices per workgroup (2 or 4): argmax, whole k-tiles");
+    static_assert(!ELEM || (TAILK && !BDIRECT && PIPE == 0 && HALVES == 1), "element loads: TAILK");
     extern __shared__ __align__(16) unsigned char dl_lds_all[];
     // HALVES > 1: the workgroup is HALVES 256-thread parts ("halves" for
     // short), each running the kernel on its own K slice with its own LDS
@@ -382,6 +405,49 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
     const int64_t gcB = col0 + (lane % Cfg::LPR) * 4;
     const uint32_t offB =
         uint32_t((lane / Cfg::LPR) * N * 4 + (gcB < N ? gcB : N - 4) * 4);
+    // Element loads of k-tile t (ELEM).  A: an instruction covers two rows of
+    // 32 k, the lane's source k in its row permuted by quads as the 16-byte
+    // loads do; B: 64 columns of one k row.  One wave-uniform base per operand
+    // and k-tile, per-lane byte offsets fixed for the whole loop; rows and
+    // columns clamp into the matrix, k past K (last) reads k = K - 1
+    // (patch_tail overwrites them).
+    constexpr int NAE = ELEM ? NAI * 4 : 1, EPR = BN / 64;
+    uint32_t eoffA[NAE];
+    const int ek = (lane & 31) * 4;
+    if constexpr (ELEM) {
+#pragma unroll
+        for (int q = 0; q < NAE; ++q) {
+            const int ins = wave * NAE + q;
+            const int64_t gr = row0 + ins * 2 + (lane >> 5);
+            eoffA[q] = uint32_t(((gr < M ? gr : M - 1) - row0) * K * 4) +
+                       uint32_t(ek ^ (((ins >> 1) & 7) << 4));
+        }
+    }
+    auto issue_elem_loads = [&](int64_t t, int buf, bool last) {
+        T* adst = As0 + buf * (BM * BK);
+        T* bdst = Bs0 + buf * (BK * BN);
+        const unsigned char* ab = reinterpret_cast<const unsigned char*>(A + row0 * K + t * BK);
+        const int left = last ? int(K - t * BK) : BK;  // k in this tile
+#pragma unroll
+        for (int q = 0; q < NAE; ++q) {
+            const int ins = wave * NAE + q;
+            uint32_t off = eoffA[q];
+            if (last) {
+                const uint32_t k4 = uint32_t(ek ^ (((ins >> 1) & 7) << 4));
+                const uint32_t max4 = uint32_t(left - 1) * 4;
+                off = off - k4 + (k4 < max4 ? k4 : max4);
+            }
+            lds_load4(ab + off, adst + ins * 64);
+        }
+        const int ins0 = wave * NBI * 4;
+        const unsigned char* bb = reinterpret_cast<const unsigned char*>(B + (t * BK + ins0 / EPR) * N);
+#pragma unroll
+        for (int q = 0; q < NBI * 4; ++q) {
+            const int64_t gc = col0 + q % EPR * 64 + lane;
+            lds_load4(bb + uint32_t((gc < N ? gc : N - 1) * 4), bdst + (ins0 + q) * 64);
+            if (q % EPR == EPR - 1 && (ins0 + q) / EPR + 1 < left) bb += N * 4;
+        }
+    };
     auto b_base = [&](int q, int64_t k0) {
         return reinterpret_cast<const unsigned char*>(B + (k0 + (wave * NBI + q) * Cfg::RPI) * N);
     };
@@ -658,7 +724,9 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
             });
         }
     } else {
-    if (TAILK && t1 - 1 == t0)
+    if constexpr (ELEM)
+        issue_elem_loads(t0, 0, t0 + 1 == t1);
+    else if (TAILK && t1 - 1 == t0)
         issue_tail_loads(t0, 0);
     else
         issue_loads(t0, 0);
@@ -667,12 +735,17 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (t + 1 < t1) {
-            if (TAILK && t + 2 == t1)
+            if constexpr (ELEM) {
+                if (t + 2 == t1)
+                    issue_elem_loads(t + 1, buf ^ 1, true);
+                else
+                    issue_elem_loads(t + 1, buf ^ 1, false);
+            } else if (TAILK && t + 2 == t1)
                 issue_tail_loads(t + 1, buf ^ 1);
             else
                 issue_loads(t + 1, buf ^ 1);
         }
-        if (TAILK && t + 1 == t1) {
+        if (TAILK && t + 1 == t1 && (!ELEM || kv < BK)) {
             patch_tail(buf, kv);
             __syncthreads();
         }
@@ -697,7 +770,18 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
 #pragma unroll
         for (int g = 0; g < TN / 4; ++g) {
             const int64_t gc = col0 + g * 64 + tx * 4;
-            if (gc >= N) continue;  // N is a multiple of 4: whole groups only
+            if (gc >= N) continue;
+            if constexpr (ELEM) {
+                if (gc + 4 > N) {  // the ragged last group
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (gc + e >= N) continue;
+                        C[gr * N + gc + e] = v[g * 4 + e];
+                        if constexpr (ARGMAX) IDX[gr * N + gc + e] = ix[g * 4 + e];
+                    }
+                    continue;
+                }
+            }  // otherwise N is a multiple of 4: whole groups only
             Vec16<T> cv;
 #pragma unroll
             for (int e = 0; e < 4; ++e) cv.v[e] = v[g * 4 + e];
@@ -917,7 +1001,14 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
             uint32_t bits = 0;
 #pragma unroll
             for (int kk = 0; kk < CL; ++kk) bits |= (p[kk] == mx) ? (1u << kk) : 0u;
-            const int f = bits ? int(__builtin_ctz(bits)) : 0;
+            int f = bits ? int(__builtin_ctz(bits)) : 0;
+            if constexpr (ELEM) {
+                // A quad that straddles K was read shifted back (its first
+                // elements belong to the quad before, and never match here
+                // unless that quad did).
+                const int64_t past = int64_t(chs[int(list[e])]) * CL + (f & ~3) - (K - 4);
+                if (past > 0) f = f - int(past) > 0 ? f - int(past) : 0;
+            }
             int r = f;
             if constexpr (std::is_floating_point<T>::value) {
                 if (mx == T(0)) {
