@@ -16,6 +16,7 @@
 
 #include "../../include/tropical_gemm_hip.h"
 #include "tg_backward.hpp"
+#include "tg_dl64s.hpp"
 #include "tg_gemm_dl.hpp"
 #include "tg_gemm_dl64.hpp"
 #include "tg_gemm_kres.hpp"
@@ -238,16 +239,14 @@ size_t dl64_ws_bytes(int64_t batch, int64_t M, int64_t N, int64_t K, bool argmax
            round_up(size_t(batch) * size_t(M + N) * 4, 256);
 }
 
-// f64, large problems (tg_gemm_dl64): the operand class prepass and, with
-// argmax, B^T staging; then the GEMM.  K % 32 == 0 and the rest of dl64_fits
-// hold.
-template <int SR>
-int run_gemm_dl64(const Problem& p, void* ws, hipStream_t st) {
-    using Cfg = tg::Dl64Cfg;
-    const int64_t tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM;
-    const int64_t tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
-    if (tiles_m * tiles_n > 0x7fffffffLL)
-        return fail(TG_ERR_DIMENSION_MISMATCH, "output too large for one launch");
+// Prepasses of the f64 direct-to-LDS kernels, into a workspace of
+// dl64_ws_bytes: operand classes and, with argmax, B^T.
+struct Dl64Ws {
+    double* BT;
+    uint32_t *clsA, *clsB;
+};
+
+int prepare_dl64(const Problem& p, void* ws, hipStream_t st, Dl64Ws* out) {
     if ((p.K + 31) / 32 > 65535 || (p.K + 255) / 256 > 65535)
         return fail(TG_ERR_DIMENSION_MISMATCH, "K too large for the staging grids");
     const double* A = static_cast<const double*>(p.A);
@@ -283,6 +282,27 @@ int run_gemm_dl64(const Problem& p, void* ws, hipStream_t st) {
                                                 cols_in_transpose ? clsB + z0 * p.N : nullptr);
         if (rc != TG_OK) return rc;
     }
+    *out = Dl64Ws{BT, clsA, clsB};
+    return TG_OK;
+}
+
+// f64, large problems (tg_gemm_dl64): the prepasses, then the GEMM.
+// K % 32 == 0 and the rest of dl64_fits hold.
+template <int SR>
+int run_gemm_dl64(const Problem& p, void* ws, hipStream_t st) {
+    using Cfg = tg::Dl64Cfg;
+    const int64_t tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM;
+    const int64_t tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
+    if (tiles_m * tiles_n > 0x7fffffffLL)
+        return fail(TG_ERR_DIMENSION_MISMATCH, "output too large for one launch");
+    Dl64Ws w;
+    const int rc = prepare_dl64(p, ws, st, &w);
+    if (rc != TG_OK) return rc;
+    const double* A = static_cast<const double*>(p.A);
+    const double* B = static_cast<const double*>(p.B);
+    const bool argmax = p.IDX != nullptr;
+    double* const BT = w.BT;
+    uint32_t *const clsA = w.clsA, *const clsB = w.clsB;
     KernelTimer timer(st);
     for (int64_t z0 = 0; z0 < p.batch; z0 += 65535) {
         const int64_t nb = (p.batch - z0 < 65535) ? p.batch - z0 : 65535;
@@ -300,6 +320,35 @@ int run_gemm_dl64(const Problem& p, void* ws, hipStream_t st) {
                                int(tiles_n));
         TG_HIP(hipGetLastError());
     }
+    return TG_OK;
+}
+
+// 64-bit problems on 64 x 64 tiles (tg_gemm_dl64s; tg::dl64s_fits holds): f64
+// with its prepasses, i64 with B^T staging for argmax.
+template <int SR, typename T>
+int run_gemm_dl64s(const Problem& p, void* ws, hipStream_t st) {
+    constexpr bool f64 = std::is_same<T, double>::value;
+    Dl64Ws w{nullptr, nullptr, nullptr};
+    T* BT = nullptr;
+    if constexpr (f64) {
+        const int rc = prepare_dl64(p, ws, st, &w);
+        if (rc != TG_OK) return rc;
+        BT = w.BT;
+    } else if (p.IDX != nullptr) {
+        if ((p.K + 31) / 32 > 65535)
+            return fail(TG_ERR_DIMENSION_MISMATCH, "K too large for the transpose grid");
+        BT = static_cast<T*>(ws);
+        for (int64_t z0 = 0; z0 < p.batch; z0 += 65535) {
+            const int64_t nb = (p.batch - z0 < 65535) ? p.batch - z0 : 65535;
+            const int rc = launch_transpose<T>(static_cast<const T*>(p.B) + z0 * p.sB,
+                                               BT + z0 * p.K * p.N, p.K, p.N, p.sB, p.K * p.N, nb, st);
+            if (rc != TG_OK) return rc;
+        }
+    }
+    KernelTimer timer(st);
+    TG_HIP(tg::dl64s_launch(tg::Dl64sProblem{SR, f64, p.A, p.B, BT, p.C, p.IDX, w.clsA, w.clsB,
+                                             p.batch, p.M, p.N, p.K, p.sA, p.sB, p.sC},
+                            st));
     return TG_OK;
 }
 
@@ -742,6 +791,18 @@ constexpr int64_t exact_tiles_max_k() {
     return sizeof(T) == 4 ? 384 : std::is_same<T, int64_t>::value ? 2048 : 512;
 }
 
+// i64 argmax leaves the exact mode earlier where its chunked tiles run
+// tg_gemm_dl64s: from K = 97 on tiles at least half full, with the workspace
+// for B^T (us on MI355X, chunked / exact: 4096^2 x 128 429 / 548, 3001^2 x
+// 300 501 / 731, 2048^3 1159 / 2047; 2048^2 x 80 122 / 95).  Batches of small
+// products would mostly stage B^T.
+template <typename T>
+bool chunked_i64(const Problem& p, size_t ws_bytes) {
+    if (!std::is_same<T, int64_t>::value || p.K <= 96 || p.M < 32 || p.N < 32) return false;
+    return ws_layout(TG_I64, p.batch, p.M, p.N, p.K, true, 1).total <= ws_bytes &&
+           tg::dl64s_fits(p.M, p.N, p.K);
+}
+
 // Problems with K up to these run the short-K kernel (when N % 4 == 0 and B,
 // C, IDX are 16-byte aligned).  Measured on MI355X (MaxPlus, against the
 // kernels these problems took before): f32 65536 x 2048 x K, argmax K = 8
@@ -754,7 +815,7 @@ constexpr int64_t kShortkArgmaxMaxK = 32;
 constexpr int64_t kShortkValueMaxK = 63;
 
 // The kernel a problem runs on.
-enum class Path { SHORTK, KRESW, KRES8, KRES, DL_88_32, DL_48_16, DL_48_VALUE, DL_44_8, DL_44_16, DL_44_32, DL_ELEM_8, DL_ELEM_16, DL_ELEM, DL64, DL64_VALUE, TILES_EXACT, TILES_CHUNKED, TILES };
+enum class Path { SHORTK, KRESW, KRES8, KRES, DL_88_32, DL_48_16, DL_48_VALUE, DL_44_8, DL_44_16, DL_44_32, DL_ELEM_8, DL_ELEM_16, DL_ELEM, DL64, DL64_VALUE, DL64S, DL64S_VALUE, TILES_EXACT, TILES_CHUNKED, TILES };
 
 struct Plan {
     Path path = Path::TILES;
@@ -774,7 +835,9 @@ bool uses_workspace(const Plan& pl, bool argmax) {
         case Path::TILES: return false;
         case Path::TILES_CHUNKED:
         case Path::DL64:
-        case Path::DL64_VALUE: return true;
+        case Path::DL64_VALUE:
+        case Path::DL64S:
+        case Path::DL64S_VALUE: return true;
         default: return argmax || pl.splits > 1;
     }
 }
@@ -913,23 +976,34 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
         }
     }
     if constexpr (std::is_same<T, double>::value) {
-        // f64 on at least 256 tiles of 64 x 128 with the workspace for the
-        // operand classes (and B^T with argmax): argmax beyond the exact
-        // range, value-only from K = 256 (below that the class prepass and
-        // its launches weigh on the product).
+        // f64 from K = 256 with the workspace for the operand classes (and B^T
+        // with argmax); below that the prepasses and their launches weigh on
+        // the product.  64 x 128 tiles where they give every CU two (argmax
+        // beyond the exact range, which they were measured against);
+        // otherwise 64 x 64 tiles of any alignment from a quarter of the CUs
+        // up (us on MI355X, against 64 x 128 tiles or the generic kernel):
+        // argmax 1536^2 x 768 245 / 357, 1024^3 149 / 277, 2047 x 2049 x 1025
+        // 518 / 1053, 3001^2 x 300 376 / 459, 3000 x 2000 x 256 221 / 250;
+        // value-only 1536^2 x 768 200 / 263, 1024^3 111 / 203, 3001^2 x 300
+        // 249 / 323.
         const int64_t tiles = ((p.M + tg::Dl64Cfg::BM - 1) / tg::Dl64Cfg::BM) *
                               ((p.N + tg::Dl64Cfg::BN - 1) / tg::Dl64Cfg::BN) * p.batch;
-        const bool deep = argmax ? !exact && p.K > exact_tiles_max_k<T>() : p.K >= 256;
-        if (deep && tiles >= 256 &&
-            tg::dl64_fits(p.M, p.N, p.K, p.sA, p.sB, p.sC, p.A, p.B, p.C, p.IDX) &&
-            dl64_ws_bytes(p.batch, p.M, p.N, p.K, argmax) <= ws_bytes) {
-            pl.path = argmax ? Path::DL64 : Path::DL64_VALUE;
-            return pl;
+        const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
+        if (p.K >= 256 && dl64_ws_bytes(p.batch, p.M, p.N, p.K, argmax) <= ws_bytes) {
+            if (tiles >= 512 && (!argmax || p.K > exact_tiles_max_k<T>()) &&
+                tg::dl64_fits(p.M, p.N, p.K, p.sA, p.sB, p.sC, p.A, p.B, p.C, p.IDX)) {
+                pl.path = argmax ? Path::DL64 : Path::DL64_VALUE;
+                return pl;
+            }
+            if (tiles64 >= 64 && tg::dl64s_fits(p.M, p.N, p.K)) {
+                pl.path = argmax ? Path::DL64S : Path::DL64S_VALUE;
+                return pl;
+            }
         }
     }
     if (!argmax)
         pl.path = Path::TILES;
-    else if (exact || p.K <= exact_tiles_max_k<T>())
+    else if (exact || (p.K <= exact_tiles_max_k<T>() && !chunked_i64<T>(p, ws_bytes)))
         pl.path = Path::TILES_EXACT;
     else
         pl.path = Path::TILES_CHUNKED;
@@ -942,6 +1016,16 @@ int run_gemm_typed(const Problem& p, void* ws, size_t ws_bytes, hipStream_t st) 
     if (pl.path == Path::SHORTK) return run_gemm_shortk<SR, T>(p, st);
     if constexpr (std::is_same<T, double>::value) {
         if (pl.path == Path::DL64 || pl.path == Path::DL64_VALUE) return run_gemm_dl64<SR>(p, ws, st);
+        if (pl.path == Path::DL64S || pl.path == Path::DL64S_VALUE)
+            return run_gemm_dl64s<SR, double>(p, ws, st);
+    }
+    if constexpr (std::is_same<T, int64_t>::value) {
+        // The chunked and the value-only tiles of i64 are tg_gemm_dl64s; the
+        // register-staged kernel keeps sizes it does not fit and value-only
+        // K below 64 (2048^2 x 80: 52 us both).
+        if ((pl.path == Path::TILES_CHUNKED || (pl.path == Path::TILES && p.K >= 64)) &&
+            tg::dl64s_fits(p.M, p.N, p.K))
+            return run_gemm_dl64s<SR, int64_t>(p, ws, st);
     }
     if constexpr (sizeof(T) == 4) {
         switch (pl.path) {
@@ -1085,6 +1169,8 @@ const char* path_name(Path path) {
         case Path::DL_ELEM: return "dl_elem";
         case Path::DL64: return "dl64_4x8_cl16";
         case Path::DL64_VALUE: return "dl64_4x8";
+        case Path::DL64S: return "dl64s_4x4_cl16";
+        case Path::DL64S_VALUE: return "dl64s_4x4";
         case Path::TILES_EXACT: return "tiles_exact";
         case Path::TILES_CHUNKED: return "tiles_chunked";
         case Path::TILES: return "tiles";
@@ -1218,10 +1304,11 @@ int gemm_impl(int device, tg_semiring sr, tg_dtype dt, tg_layout layout, const v
             const Plan pl = plan_gemm(sr, dt, p, ws_bytes);
             if (!uses_workspace(pl, with_argmax)) {
                 ws_bytes = 0;
-            } else if (pl.path == Path::DL_ELEM_8 &&
+            } else if ((pl.path == Path::DL_ELEM_8 || pl.path == Path::TILES_CHUNKED ||
+                        pl.path == Path::DL64S || pl.path == Path::DL64S_VALUE) &&
                        !uses_workspace(plan_gemm(sr, dt, p, 0), with_argmax)) {
-                // Under capture a product that can do without a workspace
-                // stays free of allocation nodes.
+                // Under capture a product that these paths took from a kernel
+                // without a workspace goes back to it: no allocation nodes.
                 hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
                 if (hipStreamIsCapturing(st, &cap) != hipSuccess) (void)hipGetLastError();
                 if (cap != hipStreamCaptureStatusNone) ws_bytes = 0;
@@ -1260,10 +1347,12 @@ tg::SmallProblem small_problem(tg_semiring sr, tg_dtype dt, const Problem& p) {
 //     999 f32 104 / 114, 7 x (500 x 501 x 502) 88 / 74; value-only 81 / 87, 57 / 44.
 //   generic tiles, 32-bit (few tiles, or K <= 96): 42 x (452 x 92 x 52) f32
 //     argmax 23 / 28, 2001^2 x 60 45 / 41.
-//   f64: 1024^3 argmax 203 / 271, value-only 143 / 202; argmax with K < 256 at
-//     100%..130% from half a million outputs (the exact mode there has
-//     no window loads).
-//   i64: 1024^3 argmax 198 / 260, 4 x (480 x 5084 x 428) 906 / 1093.
+//   f64: 700^3 argmax 79 / 111, value-only 54 / 78, 1024^3 207 / 149, 147 / 111;
+//     argmax with K < 256 at 100%..130% from half a million outputs (the exact
+//     mode there has no window loads).
+//   i64: argmax 1536^2 x 768 340 / 365, 2047 x 2049 x 1025 780 / 803, 2048^3
+//     1490 / 1160, in the exact mode's range 2048^2 x 80 83 / 95; value-only
+//     2047 x 2049 x 1025 586 / 652, 3001^2 x 300 388 / 349.
 int64_t small_output_limit(tg_dtype dt, const Plan& pl, const Problem& p) {
     constexpr int64_t k1 = int64_t(1) << 10;
     const bool argmax = p.IDX != nullptr;
@@ -1280,6 +1369,8 @@ int64_t small_output_limit(tg_dtype dt, const Plan& pl, const Problem& p) {
         case Path::KRES: return dt == TG_I32 ? 256 * k1 : 512 * k1;
         case Path::DL64:
         case Path::DL64_VALUE: return 2048 * k1;
+        case Path::DL64S:
+        case Path::DL64S_VALUE: return narrow <= 32 ? 2048 * k1 : 768 * k1;
         case Path::TILES_EXACT:
         case Path::TILES_CHUNKED:
         case Path::TILES: break;
@@ -1290,7 +1381,8 @@ int64_t small_output_limit(tg_dtype dt, const Plan& pl, const Problem& p) {
         default:  // direct-to-LDS, 32-bit
             return narrow <= 32 ? 2048 * k1 : p.K >= 256 ? 896 * k1 : 512 * k1;
     }
-    if (dt == TG_I64) return argmax ? 8192 * k1 : 4096 * k1;
+    if (dt == TG_I64)
+        return pl.path == Path::TILES_EXACT ? 8192 * k1 : 4096 * k1;
     if (dt == TG_F64) {
         if (!argmax || pl.path == Path::TILES_CHUNKED) return 2048 * k1;
         return p.K < 256 ? 512 * k1 : 1536 * k1;
@@ -1353,7 +1445,8 @@ size_t scratch_need(tg_dtype dt, const Problem& p, const Plan& pl) {
     if (!uses_workspace(pl, argmax)) return 0;
     // The f64 direct-to-LDS kernel's workspace: B^T (argmax) and the operand
     // classes of A's rows and B's columns (run_gemm_dl64).
-    if (pl.path == Path::DL64 || pl.path == Path::DL64_VALUE)
+    if (pl.path == Path::DL64 || pl.path == Path::DL64_VALUE || pl.path == Path::DL64S ||
+        pl.path == Path::DL64S_VALUE)
         return dl64_ws_bytes(p.batch, p.M, p.N, p.K, argmax);
     return ws_layout(dt, p.batch, p.M, p.N, p.K, argmax, pl.splits).total;
 }

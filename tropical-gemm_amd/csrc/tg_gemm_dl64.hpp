@@ -78,7 +78,7 @@ __device__ __forceinline__ bool nan_danger(uint32_t ca, uint32_t cb) {
 // gets them from the B^T transpose, which reads B anyway), in segments of 64
 // columns x 256 k, 4 k-lanes per column.  Both arrays zeroed beforehand.
 // Grid-stride over rows and segments; block = 256.
-__global__ __launch_bounds__(256) void tg_class_prepass(const double* __restrict__ A, int64_t M,
+static __global__ __launch_bounds__(256) void tg_class_prepass(const double* __restrict__ A, int64_t M,
                                                         int64_t K, int64_t sA,
                                                         const double* __restrict__ B, int64_t N,
                                                         int64_t sB, int64_t batch,
