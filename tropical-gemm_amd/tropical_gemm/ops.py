@@ -31,12 +31,19 @@ def as_tensor(x) -> torch.Tensor:
     raise TypeError(f"expected a tensor or a DLPack producer, got {type(x).__name__}")
 
 
-def _stream(dev: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+# The current stream's handle without building a torch.cuda.Stream object
+# (0.07 against 1.8 us; a small product's whole call takes 10).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
-def _ptr(t: torch.Tensor | None) -> ctypes.c_void_p | None:
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+def _stream(dev: torch.device) -> int:
+    if _raw_stream is not None:
+        return _raw_stream(dev.index)
+    return torch.cuda.current_stream(dev).cuda_stream
+
+
+def _ptr(t: torch.Tensor | None) -> int | None:
+    return None if t is None else t.data_ptr()
 
 
 def _check_pair(a: torch.Tensor, b: torch.Tensor, ndim: int) -> None:
@@ -65,9 +72,8 @@ def _product(semiring: str, a, b, c, am, batch: int, m: int, n: int, k: int) -> 
     dev = a.device
     dt = nat.DTYPE[_DT[a.dtype]]
     args = (dev.index or 0, nat.SEMIRING[semiring], dt, nat.LAYOUT["row"], a.data_ptr(),
-            b.data_ptr(), c.data_ptr(), None if am is None else am.data_ptr(), batch, m, n, k,
-            m * k, k * n, m * n)
-    stream = torch.cuda.current_stream(dev).cuda_stream
+            b.data_ptr(), c.data_ptr(), _ptr(am), batch, m, n, k, m * k, k * n, m * n)
+    stream = _stream(dev)
     ran = ctypes.c_int(0)
     nat.check(lib.tg_gemm_small(*args, stream, ran))
     if ran.value:
