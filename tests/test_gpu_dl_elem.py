@@ -14,10 +14,11 @@ pytestmark = pytest.mark.gpu
 
 # (m, n, k): a last k-tile of 1, 2, 3, 31 and 32 k, a last chunk of 1, 2, 3
 # and 5 k (windows that shift back over K), one row or column past a tile,
-# a last column group of 1, 2 and 3 columns, K on both sides of the chunk
-# lengths' boundary (512).
+# a last column group of 1, 2 and 3 columns; K slices of unequal length (17
+# and 18 k-tiles) and a fourth slice left empty (9 k-tiles).
 SHAPES = [(513, 511, 97), (449, 577, 130), (640, 450, 99), (576, 514, 255), (511, 513, 160),
-          (577, 449, 197), (512, 515, 511), (515, 512, 514), (513, 513, 549)]
+          (577, 449, 197), (512, 515, 511), (515, 512, 514), (513, 513, 549), (513, 512, 257),
+          (512, 577, 288), (449, 451, 1027), (512, 512, 260)]
 
 
 @pytest.mark.parametrize("dt", ["f32", "i32"])
@@ -28,8 +29,12 @@ def test_element_loads_edges(dt, m, n, k):
     rng = np.random.default_rng(m + 3 * n + 7 * k)
     dtype = tc.NP_DTYPES[dt]
     for sr in tc.SEMIRINGS:
-        assert nat.gemm_plan(sr, dt, m, n, k, True) == ("dl_elem_cl8" if k <= 512 else "dl_elem_cl16")
-        assert nat.gemm_plan(sr, dt, m, n, k, False) == "dl_elem"
+        # Up to 256 tiles, K from 256 runs in two (1024: four) slices, value-only in
+        # four.
+        cut = k >= 256
+        assert nat.gemm_plan(sr, dt, m, n, k, True) == (
+            "dl_elem_cl8" + (" slices 4" if k >= 1024 else " slices 2" if cut else ""))
+        assert nat.gemm_plan(sr, dt, m, n, k, False) == "dl_elem" + (" slices 4" if cut else "")
         # Ties across k, and winners in the last, partial window.
         lo, hi = (1, 50) if sr == "maxmul" else (-50, 50)
         a = rng.integers(lo, hi, size=(m, k))
@@ -47,9 +52,31 @@ def test_element_loads_edges(dt, m, n, k):
         np.testing.assert_array_equal(c, c_ref)
 
 
+@pytest.mark.parametrize("sr,m,n,k,with_argmax,plan", [
+    ("maxplus", 1473, 1501, 517, True, "dl_elem_cl16"),
+    ("minplus", 1090, 1201, 515, True, "dl_elem_cl8 slices 2"),
+    ("maxplus", 1090, 1200, 515, False, "dl_elem slices 2"),
+    ("maxmul", 1200, 1200, 700, True, "dl_elem_cl8 slices 2"),  # aligned
+    ("minplus", 2100, 2101, 259, False, "dl_elem"),
+])
+def test_element_loads_more_tiles(sr, m, n, k, with_argmax, plan):
+    from tropical_gemm import _native as nat
+
+    rng = np.random.default_rng(m + k)
+    a = rng.integers(1, 60, size=(m, k)).astype(np.float32)
+    b = rng.integers(1, 60, size=(k, n)).astype(np.float32)
+    rows = np.unique(np.concatenate([np.arange(0, m, 41), [63, 64, m - 1]]))
+    c_ref, am_ref = oracle.gemm(sr, a[rows], b)
+    assert nat.gemm_plan(sr, "f32", m, n, k, with_argmax) == plan
+    print(f"[case] element loads {plan} {sr} {m}x{n}x{k}", flush=True)
+    c, am = gpu_gemm(sr, a, b, with_argmax)
+    assert_exact(c[rows], am[rows] if with_argmax else None, c_ref, am_ref if with_argmax else None)
+
+
+@pytest.mark.parametrize("k", [131, 515])
 @pytest.mark.parametrize("sr", tc.SEMIRINGS)
-def test_element_loads_nan_rule_and_layouts(sr):
-    m, n, k = 513, 515, 131
+def test_element_loads_nan_rule_and_layouts(sr, k):
+    m, n = 513, 515
     a, b = nan_inputs(sr, np.float32, m, n, k, seed=3)
     c_ref, am_ref = oracle.gemm(sr, a, b)
     for layout in ("row", "col"):
@@ -81,5 +108,5 @@ def test_short_k_without_workspace_keeps_the_exact_mode():
     from tropical_gemm import _native as nat
 
     m, n, k = 513, 80001, 300
-    assert nat.gemm_plan("maxplus", "f32", m, n, k, True) == "dl_elem_cl8"
+    assert nat.gemm_plan("maxplus", "f32", m, n, k, True).startswith("dl_elem_cl8")
     assert nat.gemm_plan("maxplus", "f32", m, n, k, True, workspace_bytes=64 << 20) == "tiles_exact"

@@ -17,6 +17,7 @@
 #include "../../include/tropical_gemm_hip.h"
 #include "tg_backward.hpp"
 #include "tg_dl64s.hpp"
+#include "tg_dl_elem.hpp"
 #include "tg_gemm_dl.hpp"
 #include "tg_gemm_dl64.hpp"
 #include "tg_gemm_kres.hpp"
@@ -552,38 +553,27 @@ int run_gemm_dl(const Problem& p, void* ws, int splits, hipStream_t st) {
 }
 
 // Direct-to-LDS kernel with element loads (32-bit types; N, K, strides and
-// pointers of any alignment), 64 x 64 tiles, unsplit.  With argmax the
-// workspace holds B^T.
-template <int SR, typename T, bool ARGMAX, int CL>
-int run_gemm_dl_elem(const Problem& p, void* ws, hipStream_t st) {
-    using Cfg = tg::DlCfg<4, 4>;
-    const int64_t tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM;
-    const int64_t tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
-    if (tiles_m * tiles_n > 0x7fffffffLL)
+// pointers of any alignment), 64 x 64 tiles, K in `slices` slices per
+// workgroup.  With argmax the workspace holds B^T.
+template <int SR, typename T>
+int run_gemm_dl_elem(const Problem& p, int cl, int slices, void* ws, hipStream_t st) {
+    const bool argmax = p.IDX != nullptr;
+    if (((p.M + 63) / 64) * ((p.N + 63) / 64) > 0x7fffffffLL)
         return fail(TG_ERR_DIMENSION_MISMATCH, "output too large for one launch");
-    if (ARGMAX && (p.K + 31) / 32 > 65535)
+    if (argmax && (p.K + 31) / 32 > 65535)
         return fail(TG_ERR_DIMENSION_MISMATCH, "K too large for the transpose grid");
-    T* const BT = ARGMAX ? static_cast<T*>(ws) : nullptr;
+    T* const BT = argmax ? static_cast<T*>(ws) : nullptr;
     const int64_t sBT = p.K * p.N;
-    const T* A = static_cast<const T*>(p.A);
-    const T* B = static_cast<const T*>(p.B);
-    T* C = static_cast<T*>(p.C);
-    for (int64_t z0 = 0; ARGMAX && z0 < p.batch; z0 += 65535) {
+    for (int64_t z0 = 0; argmax && z0 < p.batch; z0 += 65535) {
         const int64_t nb = (p.batch - z0 < 65535) ? p.batch - z0 : 65535;
-        const int rc = launch_transpose<T>(B + z0 * p.sB, BT + z0 * sBT, p.K, p.N, p.sB, sBT, nb, st);
+        const int rc = launch_transpose<T>(static_cast<const T*>(p.B) + z0 * p.sB, BT + z0 * sBT, p.K,
+                                           p.N, p.sB, sBT, nb, st);
         if (rc != TG_OK) return rc;
     }
     KernelTimer timer(st);
-    for (int64_t z0 = 0; z0 < p.batch; z0 += 65535) {
-        const int64_t nb = (p.batch - z0 < 65535) ? p.batch - z0 : 65535;
-        dim3 grid(unsigned(tiles_m * tiles_n), 1, unsigned(nb));
-        hipLaunchKernelGGL((tg::tg_gemm_dl<SR, T, ARGMAX, 4, 4, CL, true, false, 0, 1, true>), grid,
-                           dim3(256), ARGMAX ? Cfg::LDS_BYTES : Cfg::TILE_BYTES, st, A + z0 * p.sA,
-                           B + z0 * p.sB, ARGMAX ? BT + z0 * sBT : nullptr, C + z0 * p.sC,
-                           ARGMAX ? p.IDX + z0 * p.sC : nullptr, p.M, p.N, p.K, p.sA, p.sB, p.sC,
-                           int(tiles_m), int(tiles_n), p.K, int64_t(0));
-        TG_HIP(hipGetLastError());
-    }
+    TG_HIP(tg::dl_elem_launch(tg::DlElemProblem{SR, std::is_same<T, float>::value, p.A, p.B, BT, p.C,
+                                                p.IDX, p.batch, p.M, p.N, p.K, p.sA, p.sB, p.sC},
+                              cl, slices, st));
     return TG_OK;
 }
 
@@ -820,6 +810,7 @@ enum class Path { SHORTK, KRESW, KRES8, KRES, DL_88_32, DL_48_16, DL_48_VALUE, D
 struct Plan {
     Path path = Path::TILES;
     int splits = 1;
+    int slices = 1;  // K slices per workgroup of the element-load paths
 };
 
 // True when the path reads the workspace: B^T staging for the resolve of the
@@ -877,6 +868,35 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
         // direct-to-LDS kernel's padded last k-tile would be wasted work;
         // the generic kernel bounds its last tile instead.
         const bool short_tail = !argmax && p.K % 32 != 0 && p.K < 64;
+        // The direct-to-LDS kernel with element loads (any N, K, strides and
+        // pointers), from a quarter of the CUs' worth of tiles up.  Measured
+        // on MI355X against the generic kernel (us): argmax 2001^3 f32 348 /
+        // 750, i32 455 / 807, 701^3 54 / 301, 3001 x 1501 x 301 102 / 182,
+        // 3001^2 x 100 104 / 121, x 65 91 / 86 (so up to K = 96 the exact mode
+        // stays); value-only 2001^3 291 / 342, 2001^2 x 60 15.5 / 22.8.  Below
+        // K = 48 most of a second k-tile would be padding.
+        const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
+        const int slices = tg::dl_elem_slices(tiles64, p.K, argmax);
+        auto take_elem = [&]() {
+            if (tiles64 < 64 || !tg::dl_elem_fits<8>(p.M, p.N, p.K)) return false;
+            if (!argmax) {
+                if (p.K < 48) return false;
+                pl.path = Path::DL_ELEM;
+            } else {
+                const tg_dtype dt = std::is_same<T, float>::value ? TG_F32 : TG_I32;
+                if (p.K <= kExactPartialMaxK ||
+                    ws_layout(dt, p.batch, p.M, p.N, p.K, true, 1).total > ws_bytes)
+                    return false;
+                pl.path = slices > 1 || p.K <= 512 ? Path::DL_ELEM_8 : Path::DL_ELEM_16;
+            }
+            pl.slices = slices;
+            return true;
+        };
+        // Aligned problems of up to two tiles per CU whose K the kernels below
+        // do not split: its K slices outweigh the element loads (1300^3 f32
+        // argmax 134 / 137 us, 4000 x 300 x 2000 180 / 187, 1200 x 1300 x 700
+        // 82 / 89; value-only 94 / 104, 135 / 158, 52 / 58).
+        if (slices > 1 && tiles64 <= 512 && (tiles64 > 256 || p.K % 64 != 0) && take_elem()) return pl;
         if (!exact && !short_tail && !(partial && argmax && p.K <= kExactPartialMaxK)) {
             // Direct-to-LDS kernels (value-only, or argmax beyond the exact
             // range).  Split K when the problem makes too few 64 x 64 tiles
@@ -953,27 +973,7 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
             }
             pl.splits = 1;
         }
-        // Rows or operands that are not whole 16-byte vectors: the
-        // direct-to-LDS kernel with element loads, from a quarter of the
-        // CUs' worth of tiles up.  Measured on MI355X against the generic
-        // kernel (us): argmax 2001^3 f32 348 / 750, i32 455 / 807, 701^3 75 /
-        // 301, 3001 x 1501 x 301 102 / 182, 3001^2 x 100 104 / 121, x 65
-        // 91 / 86 (so up to K = 96 the exact mode stays); value-only 2001^3
-        // 291 / 342, 2001^2 x 60 15.5 / 22.8.  Below K = 48 most of a second
-        // k-tile would be padding.
-        const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
-        if (tiles64 >= 64 && tg::dl_elem_fits<8>(p.M, p.N, p.K)) {
-            if (!argmax && p.K >= 48) {
-                pl.path = Path::DL_ELEM;
-                return pl;
-            }
-            const tg_dtype dt = std::is_same<T, float>::value ? TG_F32 : TG_I32;
-            if (argmax && p.K > kExactPartialMaxK &&
-                ws_layout(dt, p.batch, p.M, p.N, p.K, true, 1).total <= ws_bytes) {
-                pl.path = p.K <= 512 ? Path::DL_ELEM_8 : Path::DL_ELEM_16;
-                return pl;
-            }
-        }
+        if (take_elem()) return pl;
     }
     if constexpr (std::is_same<T, double>::value) {
         // f64 from K = 256 with the workspace for the operand classes (and B^T
@@ -1044,9 +1044,9 @@ int run_gemm_typed(const Problem& p, void* ws, size_t ws_bytes, hipStream_t st) 
             case Path::DL_44_8: return run_gemm_dl<SR, T, 4, 4, 8>(p, ws, pl.splits, st);
             case Path::DL_44_16: return run_gemm_dl<SR, T, 4, 4, 16>(p, ws, pl.splits, st);
             case Path::DL_44_32: return run_gemm_dl<SR, T, 4, 4, 32>(p, ws, pl.splits, st);
-            case Path::DL_ELEM_8: return run_gemm_dl_elem<SR, T, true, 8>(p, ws, st);
-            case Path::DL_ELEM_16: return run_gemm_dl_elem<SR, T, true, 16>(p, ws, st);
-            case Path::DL_ELEM: return run_gemm_dl_elem<SR, T, false, 32>(p, ws, st);
+            case Path::DL_ELEM_8:
+            case Path::DL_ELEM: return run_gemm_dl_elem<SR, T>(p, 8, pl.slices, ws, st);
+            case Path::DL_ELEM_16: return run_gemm_dl_elem<SR, T>(p, 16, pl.slices, ws, st);
             default: break;
         }
     }
@@ -1341,10 +1341,11 @@ tg::SmallProblem small_problem(tg_semiring sr, tg_dtype dt, const Problem& p) {
 //     672 x 16 9.7 / 7.5; value-only 800 x 672 x 16 5.4 / 6.8, 368 x 4848 x 16
 //     7.7 / 6.6.  Their 256-column tiles are mostly padding for narrow N:
 //     262144 x 16 x 16 argmax 29 / 114.
-//   direct-to-LDS and K-resident (32-bit, aligned): 900^3 f32 argmax 62 / 91,
+//   direct-to-LDS and K-resident (32-bit, aligned): 768^3 f32 argmax 39 / 49,
 //     1024^3 84 / 59; i32 5376 x 64 x 64 9.6 / 9.5.
-//   direct-to-LDS with element loads (32-bit, unaligned): argmax 1531 x 777 x
-//     999 f32 104 / 114, 7 x (500 x 501 x 502) 88 / 74; value-only 81 / 87, 57 / 44.
+//   direct-to-LDS with element loads (32-bit): f32 argmax 701^3 37 / 54, 734 x
+//     1071 x 3636 232 / 180, 1001^3 102 / 76; value-only 701^3 27 / 29, 734 x
+//     1071 x 3636 195 / 136 (i32 198 / 186); unsliced 1500^2 x 150 47 / 46.
 //   generic tiles, 32-bit (few tiles, or K <= 96): 42 x (452 x 92 x 52) f32
 //     argmax 23 / 28, 2001^2 x 60 45 / 41.
 //   f64: 700^3 argmax 79 / 111, value-only 54 / 78, 1024^3 207 / 149, 147 / 111;
@@ -1377,9 +1378,11 @@ int64_t small_output_limit(tg_dtype dt, const Plan& pl, const Problem& p) {
         case Path::DL_ELEM_8:
         case Path::DL_ELEM_16:
         case Path::DL_ELEM:
-            return narrow <= 32 || (argmax && p.K < 256) ? 2048 * k1 : 1280 * k1;
+            if (narrow <= 32 || (argmax && p.K < 256)) return 2048 * k1;
+            if (pl.slices == 1) return 1280 * k1;
+            return argmax ? 640 * k1 : dt == TG_F32 ? 512 * k1 : 768 * k1;
         default:  // direct-to-LDS, 32-bit
-            return narrow <= 32 ? 2048 * k1 : p.K >= 256 ? 896 * k1 : 512 * k1;
+            return narrow <= 32 ? 2048 * k1 : p.K >= 256 ? 640 * k1 : 512 * k1;
     }
     if (dt == TG_I64)
         return pl.path == Path::TILES_EXACT ? 8192 * k1 : 4096 * k1;
@@ -1958,6 +1961,8 @@ const char* tg_gemm_plan(tg_semiring semiring, tg_dtype dtype, tg_layout layout,
     const bool slices_ok = pl.path == Path::DL_44_8 || pl.path == Path::DL_44_16;
     if (const int s = wg_slices(slices_ok, argmax != nullptr, pl.splits, p.K))
         name += " slices " + std::to_string(s);
+    else if (pl.slices > 1)
+        name += " slices " + std::to_string(pl.slices);
     else if (pl.splits > 1)
         name += " split " + std::to_string(pl.splits);
     return name.c_str();

@@ -339,16 +339,19 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
     static_assert(CL == 8 || CL == 16 || CL == 32, "argmax chunk of 8, 16 or 32 k");
     static_assert(!ARGMAX || (BK / CL) % 2 == 0, "argmax: an even number of chunks per k-tile");
     static_assert(!ARGMAX || TM == 4, "argmax tiles have 4 rows per thread");
-    static_assert(HALVES == 1 || ((HALVES == 2 || HALVES == 4) && ARGMAX && !TAILK && PIPE == 0),
-                  "K slices per workgroup (2 or 4): argmax, whole k-tiles");
-    static_assert(!ELEM || (TAILK && !BDIRECT && PIPE == 0 && HALVES == 1), "element loads: TAILK");
+    static_assert(HALVES == 1 || ((HALVES == 2 || HALVES == 4) && PIPE == 0 && TN == 4 &&
+                                  (ELEM || (ARGMAX && !TAILK))),
+                  "K slices per workgroup (2 or 4): 64 x 64 tiles; 16-byte loads: argmax, whole k-tiles");
+    static_assert(!ELEM || (TAILK && !BDIRECT && PIPE == 0), "element loads: TAILK");
+    // Bytes of LDS per slice.
+    constexpr int SLICE_BYTES = ARGMAX ? Cfg::LDS_BYTES : Cfg::TILE_BYTES;
     extern __shared__ __align__(16) unsigned char dl_lds_all[];
     // HALVES > 1: the workgroup is HALVES 256-thread parts ("halves" for
     // short), each running the kernel on its own K slice with its own LDS
     // block; they meet only at the barriers (every barrier is reached by
     // all of them) and in the merge before the resolve.
     const int half = HALVES > 1 ? int(__builtin_amdgcn_readfirstlane(threadIdx.x >> 8)) : 0;
-    unsigned char* const dl_lds = dl_lds_all + (HALVES > 1 ? half * Cfg::LDS_BYTES : 0);
+    unsigned char* const dl_lds = dl_lds_all + (HALVES > 1 ? half * SLICE_BYTES : 0);
     T* const As0 = reinterpret_cast<T*>(dl_lds);
     T* const Bs0 = reinterpret_cast<T*>(dl_lds + 2 * Cfg::A_BYTES);
 
@@ -522,7 +525,7 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
     // offsets are recomputed per tile (a few VALU ops) instead of being held
     // in registers through the loop.
     int swz_t = ty & 7;
-    auto load_frag = [&](int buf, int kk, T (&a)[TM][2], T (&b)[2][TN]) {
+    auto load_frag = [&](int buf, int kk, T (&a)[TM][2], T (&b)[2][TN]) __attribute__((always_inline)) {
         const T* as = As0 + buf * (BM * BK);
         const T* bs = Bs0 + buf * (BK * BN);
         const int q = (((kk >> 2) ^ swz_t) << 2) + (kk & 3);
@@ -541,7 +544,8 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
     // buffer buf fold into a max3/min3 chain that starts from `from` and ends
     // in `to`; the chunk is recorded where `to` strictly beats `from`.
     // Value-only: the chain runs in place (from and to are the same array).
-    auto chunk = [&](int64_t t, int buf, int s, const T (&from)[TM][TN], T (&to)[TM][TN]) {
+    auto chunk = [&](int64_t t, int buf, int s, const T (&from)[TM][TN], T (&to)[TM][TN])
+                     __attribute__((always_inline)) {
 #pragma unroll
         for (int kk = s * CL; kk < (s + 1) * CL; kk += 2) {
             T a[TM][2], b[2][TN];
@@ -572,9 +576,28 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
     // k-tiles [t0, t1) of this slice; t (and so every chunk index) is global.
     // Split slices are whole k-tiles; an unsplit K may end in a partial one
     // holding kv valid k.
+    // ELEM slices in one workgroup: KS is whole k-tiles, the last slices may
+    // hold fewer or none; every slice runs the same number of rounds
+    // (barriers), the partial k-tile falling into round tail_round of its
+    // slice.
+    constexpr bool UNEVEN = ELEM && HALVES > 1;
+    const int64_t nkt = (K + BK - 1) / BK;
     const int64_t t0 = y * (KS / BK);
-    const int64_t t1 = t0 + (KS + BK - 1) / BK;
-    const int kv = TAILK ? int(KS - (t1 - 1 - t0) * BK) : BK;
+    const int64_t t1 = UNEVEN ? (t0 + KS / BK < nkt ? t0 + KS / BK : nkt) : t0 + (KS + BK - 1) / BK;
+    const int kv = UNEVEN ? int(K - (nkt - 1) * BK) : TAILK ? int(KS - (t1 - 1 - t0) * BK) : BK;
+    // Every chunk of the k-tile t in buffer buf.
+    auto tile_chunks = [&](int64_t t, int buf) __attribute__((always_inline)) {
+        if constexpr (ARGMAX) {
+#pragma unroll
+            for (int s = 0; s < BK / CL; s += 2) {
+                chunk(t, buf, s, acc, alt);
+                chunk(t, buf, s + 1, alt, acc);
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < BK / CL; ++s) chunk(t, buf, s, acc, acc);
+        }
+    };
     if constexpr (PIPE != 0) {
         static_assert(TM == 8 && TN == 8 && !TAILK && !ARGMAX,
                       "pipelined main loop: value-only 8 x 8 outputs, whole k-tiles");
@@ -724,6 +747,29 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
             });
         }
     } else {
+    if constexpr (UNEVEN) {
+        if (t0 < t1) issue_elem_loads(t0, 0, t0 + 1 == nkt);
+        const int rounds = int(KS / BK);
+        const int tail_round = kv < BK ? int((nkt - 1) % rounds) : -1;
+        for (int r = 0; r < rounds; ++r) {
+            const int64_t t = t0 + r;
+            const int buf = r & 1;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (t + 1 < t1) {
+                if (t + 2 == nkt)
+                    issue_elem_loads(t + 1, buf ^ 1, true);
+                else
+                    issue_elem_loads(t + 1, buf ^ 1, false);
+            }
+            if (r == tail_round) {
+                if (t == nkt - 1) patch_tail(buf, kv);
+                __syncthreads();
+            }
+            asm volatile("" : "+v"(swz_t));
+            if (t < t1) tile_chunks(t, buf);
+        }
+    } else {
     if constexpr (ELEM)
         issue_elem_loads(t0, 0, t0 + 1 == t1);
     else if (TAILK && t1 - 1 == t0)
@@ -750,16 +796,8 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
             __syncthreads();
         }
         asm volatile("" : "+v"(swz_t));
-        if constexpr (ARGMAX) {
-#pragma unroll
-            for (int s = 0; s < BK / CL; s += 2) {
-                chunk(t, buf, s, acc, alt);
-                chunk(t, buf, s + 1, alt, acc);
-            }
-        } else {
-#pragma unroll
-            for (int s = 0; s < BK / CL; ++s) chunk(t, buf, s, acc, acc);
-        }
+        tile_chunks(t, buf);
+    }
     }
     }
 
@@ -803,7 +841,7 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
     // The outputs to redo go through a bit mask and one runtime loop, so the
     // serial code is not unrolled per output and does not press on the main
     // loop's registers.
-    const bool split = HALVES > 1 || gridDim.y > 1;
+    const bool split = (ARGMAX && HALVES > 1) || gridDim.y > 1;
     static_assert(TM * TN <= 64, "one mask bit per output");
     uint64_t redo = 0;
     auto redo_outputs = [&](bool argmax_out) {
@@ -823,6 +861,29 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
             if (argmax_out) IDX[gr * N + gc] = ix;
         }
     };
+    if constexpr (!ARGMAX && HALVES > 1) {
+        // Join the slices (NaN-propagating: a NaN product of any slice shows).
+        T* const mv = reinterpret_cast<T*>(dl_lds);
+        static_assert(TM * TN * TG_THREADS * 4 <= SLICE_BYTES, "merge buffer fits");
+        __syncthreads();  // every wave is done with the tile buffers
+        if (half > 0) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) mv[(i * TN + j) * TG_THREADS + tid] = acc[i][j];
+        }
+        __syncthreads();
+        if (half > 0) return;
+#pragma unroll 1
+        for (int h = 1; h < HALVES; ++h) {
+            const T* const hv = reinterpret_cast<const T*>(dl_lds_all + h * SLICE_BYTES);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    acc[i][j] = tjoin<SR, T>(acc[i][j], hv[(i * TN + j) * TG_THREADS + tid]);
+        }
+    }
     if constexpr (!ARGMAX) {
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
@@ -893,7 +954,7 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
             if (half == 0) {
 #pragma unroll 1
                 for (int h = 1; h < HALVES; ++h) {
-                    const T* const mv = reinterpret_cast<const T*>(dl_lds_all + h * Cfg::LDS_BYTES);
+                    const T* const mv = reinterpret_cast<const T*>(dl_lds_all + h * SLICE_BYTES);
                     const int32_t* const mi =
                         reinterpret_cast<const int32_t*>(mv + TM * TN * TG_THREADS);
 #pragma unroll
