@@ -802,8 +802,13 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
     }
 
     // ---- epilogue ------------------------------------------------------------
+    // Rows of outputs a thread finishes: all TM of its own, or with slices,
+    // whose merge spreads the tile over every thread of the workgroup,
+    // TM / HALVES of them.
+    constexpr int ER = TM / HALVES;
+    auto erow = [&](int i) { return trow(HALVES > 1 ? half * ER + i : i); };
     auto store_row = [&](int i, const T (&v)[TN], const int32_t (&ix)[TN]) {
-        const int64_t gr = row0 + trow(i);
+        const int64_t gr = row0 + erow(i);
         if (gr >= M) return;
 #pragma unroll
         for (int g = 0; g < TN / 4; ++g) {
@@ -841,7 +846,7 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
     // The outputs to redo go through a bit mask and one runtime loop, so the
     // serial code is not unrolled per output and does not press on the main
     // loop's registers.
-    const bool split = (ARGMAX && HALVES > 1) || gridDim.y > 1;
+    const bool split = gridDim.y > 1;
     static_assert(TM * TN <= 64, "one mask bit per output");
     uint64_t redo = 0;
     auto redo_outputs = [&](bool argmax_out) {
@@ -849,7 +854,7 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
         while (redo) {
             const int o = __builtin_ctzll(redo);
             redo &= redo - 1;
-            const int64_t gr = row0 + trow(o / TN), gc = col0 + tcol(o % TN);
+            const int64_t gr = row0 + erow(o / TN), gc = col0 + tcol(o % TN);
             if (split || gr >= M || gc >= N) continue;
             T v;
             int32_t ix;
@@ -862,31 +867,31 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
         }
     };
     if constexpr (!ARGMAX && HALVES > 1) {
-        // Join the slices (NaN-propagating: a NaN product of any slice shows).
+        // Join the slices (NaN-propagating: a NaN product of any slice shows),
+        // each part of the workgroup its rows.
         T* const mv = reinterpret_cast<T*>(dl_lds);
         static_assert(TM * TN * TG_THREADS * 4 <= SLICE_BYTES, "merge buffer fits");
         __syncthreads();  // every wave is done with the tile buffers
-        if (half > 0) {
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) mv[(i * TN + j) * TG_THREADS + tid] = acc[i][j];
-        }
+            for (int j = 0; j < TN; ++j) mv[(i * TN + j) * TG_THREADS + tid] = acc[i][j];
         __syncthreads();
-        if (half > 0) return;
-#pragma unroll 1
-        for (int h = 1; h < HALVES; ++h) {
-            const T* const hv = reinterpret_cast<const T*>(dl_lds_all + h * SLICE_BYTES);
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < ER; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    acc[i][j] = tjoin<SR, T>(acc[i][j], hv[(i * TN + j) * TG_THREADS + tid]);
-        }
+            for (int j = 0; j < TN; ++j) {
+                const int o = ((half * ER + i) * TN + j) * TG_THREADS + tid;
+                T v = reinterpret_cast<const T*>(dl_lds_all)[o];
+#pragma unroll
+                for (int h = 1; h < HALVES; ++h)
+                    v = tjoin<SR, T>(v, reinterpret_cast<const T*>(dl_lds_all + h * SLICE_BYTES)[o]);
+                acc[i][j] = v;
+            }
     }
     if constexpr (!ARGMAX) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
+        for (int i = 0; i < ER; ++i) {
             int32_t none[TN] = {};
 #pragma unroll
             for (int j = 0; j < TN; ++j)
@@ -907,8 +912,8 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
         // slot, and the thread that owns the output combines them with its
         // own record.
         constexpr uint16_t NONE = 0xFFFF;
-        // Halves: the first half's block holds the one sorted list of the
-        // merged outputs; each half keeps its own scan scratch.
+        // Slices: the first one's block holds the one sorted list of the
+        // merged outputs; each slice keeps its own scan scratch.
         constexpr bool H2 = HALVES > 1;
         unsigned char* const ep_lds = H2 ? dl_lds_all : dl_lds;
         uint32_t* hist = reinterpret_cast<uint32_t*>(ep_lds + Cfg::HIST_OFF);
@@ -932,61 +937,63 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
                 if (tisnan(acc[i][j])) ch[i][j] = -2;
         __syncthreads();  // every wave is done with the tile buffers
         if constexpr (H2) {
-            // Merge the halves before the resolve, in k order as
+            // Merge the slices before the resolve, in k order as
             // tg_merge_splits does: a later slice replaces the running result
             // only if strictly better.  Only the winning slice's chunk is
-            // then resolved, by all the workgroup's threads.  An output that
-            // met a NaN product in any slice (chunk -2) is recomputed at the
-            // end.  Halves 1.. hand over through their own LDS blocks.
+            // then resolved.  An output that met a NaN product in any slice
+            // (chunk -2) is recomputed at the end.  Every slice hands its
+            // outputs over through its own LDS block, and each part of the
+            // workgroup merges, and from here on owns, its rows of the tile
+            // (one part doing it all took 1024^3 argmax to 59 us).
             static_assert(2 * TM * TN * TG_THREADS * 4 <= Cfg::LDS_BYTES, "merge buffer fits");
-            if (half > 0) {
-                T* const mv = reinterpret_cast<T*>(dl_lds);
-                int32_t* const mi = reinterpret_cast<int32_t*>(mv + TM * TN * TG_THREADS);
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) {
-                        mv[(i * TN + j) * TG_THREADS + tid] = acc[i][j];
-                        mi[(i * TN + j) * TG_THREADS + tid] = ch[i][j];
-                    }
-            }
-            __syncthreads();
-            if (half == 0) {
-#pragma unroll 1
-                for (int h = 1; h < HALVES; ++h) {
-                    const T* const mv = reinterpret_cast<const T*>(dl_lds_all + h * SLICE_BYTES);
-                    const int32_t* const mi =
-                        reinterpret_cast<const int32_t*>(mv + TM * TN * TG_THREADS);
-#pragma unroll
-                    for (int i = 0; i < TM; ++i)
-#pragma unroll
-                        for (int j = 0; j < TN; ++j) {
-                            const T v1 = mv[(i * TN + j) * TG_THREADS + tid];
-                            const int32_t c1 = mi[(i * TN + j) * TG_THREADS + tid];
-                            if (ch[i][j] == -2 || c1 == -2) {
-                                ch[i][j] = -2;
-                            } else if (tbetter<SR, T>(v1, acc[i][j])) {
-                                acc[i][j] = v1;
-                                ch[i][j] = c1;
-                            }
-                        }
-                }
-            }
-            __syncthreads();  // the merge buffers are free again
-        }
-        const bool sorter = !H2 || half == 0;
-        if (sorter && tid < Cfg::NB) hist[tid] = 0;
-        __syncthreads();
-        if (sorter) {
+            T* const mv = reinterpret_cast<T*>(dl_lds);
+            int32_t* const mi = reinterpret_cast<int32_t*>(mv + TM * TN * TG_THREADS);
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
-                    const int lid = trow(i) * BN + tcol(j);
-                    chs[lid] = ch[i][j] < 0 ? NONE : uint16_t(ch[i][j]);
-                    if (ch[i][j] >= 0) atomicAdd(&hist[ch[i][j] >> shift], 1u);
+                    mv[(i * TN + j) * TG_THREADS + tid] = acc[i][j];
+                    mi[(i * TN + j) * TG_THREADS + tid] = ch[i][j];
                 }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < ER; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const int o = ((half * ER + i) * TN + j) * TG_THREADS + tid;
+                    T v;
+                    int32_t c;
+#pragma unroll
+                    for (int h = 0; h < HALVES; ++h) {
+                        const T* const hv = reinterpret_cast<const T*>(dl_lds_all + h * SLICE_BYTES);
+                        const T v1 = hv[o];
+                        const int32_t c1 = reinterpret_cast<const int32_t*>(hv + TM * TN * TG_THREADS)[o];
+                        if (h == 0) {
+                            v = v1;
+                            c = c1;
+                        } else if (c == -2 || c1 == -2) {
+                            c = -2;
+                        } else if (tbetter<SR, T>(v1, v)) {
+                            v = v1;
+                            c = c1;
+                        }
+                    }
+                    acc[i][j] = v;
+                    ch[i][j] = c;
+                }
+            __syncthreads();  // the merge buffers are free again
         }
+        const bool sorter = !H2 || half == 0;  // scans the buckets
+        if (sorter && tid < Cfg::NB) hist[tid] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < ER; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int lid = erow(i) * BN + tcol(j);
+                chs[lid] = ch[i][j] < 0 ? NONE : uint16_t(ch[i][j]);
+                if (ch[i][j] >= 0) atomicAdd(&hist[ch[i][j] >> shift], 1u);
+            }
         __syncthreads();
         // Exclusive scan of the bucket counts; the starts become cursors.
         const int cnt = sorter && tid < nb ? int(hist[tid]) : 0;
@@ -998,14 +1005,12 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
         }
         __syncthreads();
         if constexpr (H2) total = *shared_total;
-        if (sorter) {
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < ER; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    if (ch[i][j] >= 0)
-                        list[atomicAdd(&hist[ch[i][j] >> shift], 1u)] = uint16_t(trow(i) * BN + tcol(j));
-        }
+            for (int j = 0; j < TN; ++j)
+                if (ch[i][j] >= 0)
+                    list[atomicAdd(&hist[ch[i][j] >> shift], 1u)] = uint16_t(erow(i) * BN + tcol(j));
         __syncthreads();
 
         // Resolve, chunk-sorted, one output per thread at a time, the next
@@ -1103,7 +1108,7 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
 
         // Each output's (value, first k) of this slice; acc and ch take them.
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < ER; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 int32_t ix;
@@ -1114,7 +1119,7 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
                     acc[i][j] = tzero<SR, T>();
                     ix = 0;
                 } else {
-                    const int r = chs[trow(i) * BN + tcol(j)];
+                    const int r = chs[erow(i) * BN + tcol(j)];
                     ix = ch[i][j] * CL + (r & 31);
                     if constexpr (std::is_floating_point<T>::value) {
                         if (acc[i][j] == T(0)) acc[i][j] = (r & 32) ? -T(0) : T(0);
@@ -1122,34 +1127,9 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
                 }
                 ch[i][j] = ix;
             }
-        if constexpr (H2) {
-            // The first half holds the merged outputs; a NaN in either slice
-            // is recomputed with the reference's serial rule over the whole
-            // k range (the unsplit kernel's redo, which a split slice skips).
-            if (half == 0) {
 #pragma unroll
-                for (int i = 0; i < TM; ++i) store_row(i, acc[i], ch[i]);
-#pragma unroll 1
-                while (redo) {
-                    const int o = __builtin_ctzll(redo);
-                    redo &= redo - 1;
-                    const int64_t gr = row0 + trow(o / TN), gc = col0 + tcol(o % TN);
-                    if (gr >= M || gc >= N) continue;
-                    T v;
-                    int32_t ix;
-                    if (!BDIRECT)
-                        cpu_select<SR, T>(A + gr * K, 1, BT + gc * K, 1, K, v, ix);
-                    else
-                        cpu_select<SR, T>(A + gr * K, 1, B + gc, N, K, v, ix);
-                    C[gr * N + gc] = v;
-                    IDX[gr * N + gc] = ix;
-                }
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < TM; ++i) store_row(i, acc[i], ch[i]);
-            if constexpr (std::is_floating_point<T>::value) redo_outputs(true);
-        }
+        for (int i = 0; i < ER; ++i) store_row(i, acc[i], ch[i]);
+        if constexpr (std::is_floating_point<T>::value) redo_outputs(true);
     }
 }
 

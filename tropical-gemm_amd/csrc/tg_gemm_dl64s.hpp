@@ -342,93 +342,92 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
     }
 
     // ---- merge of the slices -----------------------------------------------------
-    // In k order into the first slice: a later one replaces the running result
-    // only if strictly better.  Values first (a slice's 32 KB hold exactly
-    // them), then the records of the slice each output took.
+    // In k order: a later slice replaces the running result only if strictly
+    // better.  Values first (a slice's 32 KB hold exactly them), then the
+    // records of the slice each output took.  Each 256-thread part merges, and
+    // from here on owns, some rows of every thread's outputs: rows [er0, er0 +
+    // ern), an extra one for the first part where they do not divide.
+    constexpr int ER = (TM + HALVES - 1) / HALVES;
+    const int er0 = HALVES == 3 ? (half == 0 ? 0 : half + 1) : half * ER;
+    const int ern = HALVES == 3 && half > 0 ? 1 : ER;
     __syncthreads();  // every wave is done with the tile buffers
     if constexpr (HALVES > 1) {
         T* const mv = reinterpret_cast<T*>(lds);
-        if (half > 0) {
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) mv[(i * TN + j) * TG_THREADS + tid] = acc[i][j];
-        }
+            for (int j = 0; j < TN; ++j) mv[(i * TN + j) * TG_THREADS + tid] = acc[i][j];
         __syncthreads();
         uint32_t took = 0;  // two bits per output: the slice its result came from
-        if (half == 0) {
-#pragma unroll 1
-            for (int h = 1; h < HALVES; ++h) {
-                const T* const hv = reinterpret_cast<const T*>(dl64s_lds + h * Cfg::LDS_BYTES);
 #pragma unroll
-                for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < ER; ++i) {
+            if (i >= ern) break;
 #pragma unroll
-                    for (int j = 0; j < TN; ++j) {
-                        const int o = i * TN + j;
-                        const T v1 = hv[o * TG_THREADS + tid];
-                        if (tbetter<SR, T>(v1, acc[i][j])) {
-                            acc[i][j] = v1;
-                            took = (took & ~(3u << (2 * o))) | (uint32_t(h) << (2 * o));
-                        }
+            for (int j = 0; j < TN; ++j) {
+                const int o = ((er0 + i) * TN + j) * TG_THREADS + tid;
+                T v = reinterpret_cast<const T*>(dl64s_lds)[o];
+#pragma unroll
+                for (int g = 1; g < HALVES; ++g) {
+                    const T v1 = reinterpret_cast<const T*>(dl64s_lds + g * Cfg::LDS_BYTES)[o];
+                    if (tbetter<SR, T>(v1, v)) {
+                        v = v1;
+                        took = (took & ~(3u << (2 * (i * TN + j)))) | (uint32_t(g) << (2 * (i * TN + j)));
                     }
+                }
+                acc[i][j] = v;
             }
         }
         if constexpr (ARGMAX) {
             __syncthreads();
             int32_t* const mi = reinterpret_cast<int32_t*>(lds);
-            if (half > 0) {
 #pragma unroll
-                for (int i = 0; i < TM; ++i)
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-                    for (int j = 0; j < TN; ++j) mi[(i * TN + j) * TG_THREADS + tid] = ch[i][j];
-            }
+                for (int j = 0; j < TN; ++j) mi[(i * TN + j) * TG_THREADS + tid] = ch[i][j];
             __syncthreads();
-            if (half == 0) {
 #pragma unroll
-                for (int i = 0; i < TM; ++i)
+            for (int i = 0; i < ER; ++i) {
+                if (i >= ern) break;
 #pragma unroll
-                    for (int j = 0; j < TN; ++j) {
-                        const int o = i * TN + j;
-                        const uint32_t h = (took >> (2 * o)) & 3u;
-                        if (h)
-                            ch[i][j] = reinterpret_cast<const int32_t*>(
-                                dl64s_lds + h * Cfg::LDS_BYTES)[o * TG_THREADS + tid];
-                    }
+                for (int j = 0; j < TN; ++j) {
+                    const uint32_t g = (took >> (2 * (i * TN + j))) & 3u;
+                    ch[i][j] = reinterpret_cast<const int32_t*>(
+                        dl64s_lds + g * Cfg::LDS_BYTES)[((er0 + i) * TN + j) * TG_THREADS + tid];
+                }
             }
             __syncthreads();  // the blocks are free again
         }
     }
-    const bool owner = HALVES == 1 || half == 0;  // holds the merged outputs
 
     // ---- epilogue ------------------------------------------------------------------
     // f64 outputs whose row and column could meet in a NaN product: recomputed
     // after the stores with the serial rule.
     uint32_t redo = 0;
+    auto erow = [&](int i) { return trow(er0 + i); };
     if constexpr (F64) {
-        if (owner) {
-            uint32_t cb[TN];
+        uint32_t cb[TN];
 #pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const int64_t gc = col0 + tcol(j);
-                cb[j] = clsB[gc < N ? gc : N - 1];
-            }
+        for (int j = 0; j < TN; ++j) {
+            const int64_t gc = col0 + tcol(j);
+            cb[j] = clsB[gc < N ? gc : N - 1];
+        }
 #pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                const int64_t gr = row0 + trow(i);
-                const uint32_t ra = clsA[gr < M ? gr : M - 1];
+        for (int i = 0; i < ER; ++i) {
+            if (i >= ern) break;
+            const int64_t gr = row0 + erow(i);
+            const uint32_t ra = clsA[gr < M ? gr : M - 1];
 #pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    if (nan_danger<SR>(ra, cb[j])) {
-                        redo |= 1u << (i * TN + j);
-                        ch[i][j] = -2;
-                    }
-            }
+            for (int j = 0; j < TN; ++j)
+                if (nan_danger<SR>(ra, cb[j])) {
+                    redo |= 1u << (i * TN + j);
+                    ch[i][j] = -2;
+                }
         }
     }
     const bool vec_out = N % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15u) == 0 &&
                          (!ARGMAX || (reinterpret_cast<uintptr_t>(IDX) & 15u) == 0);
     auto store_row = [&](int i) {
-        const int64_t gr = row0 + trow(i), gc = col0 + tcol(0);
+        const int64_t gr = row0 + erow(i), gc = col0 + tcol(0);
         if (gr >= M || gc >= N) return;
         T* c = C + gr * N + gc;
         if (vec_out) {  // N a multiple of 4: whole groups only
@@ -459,7 +458,7 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
         while (redo) {
             const int o = __builtin_ctz(redo);
             redo &= redo - 1;
-            const int64_t gr = row0 + trow(o / TN), gc = col0 + tcol(o % TN);
+            const int64_t gr = row0 + erow(o / TN), gc = col0 + tcol(o % TN);
             if (gr >= M || gc >= N) continue;
             T v;
             int32_t ix;
@@ -472,11 +471,10 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
         }
     };
     if constexpr (!ARGMAX) {
-        if (owner) {
 #pragma unroll
-            for (int i = 0; i < TM; ++i) store_row(i);
-            if constexpr (F64) redo_outputs();
-        }
+        for (int i = 0; i < ER; ++i)
+            if (i < ern) store_row(i);
+        if constexpr (F64) redo_outputs();
     } else {
         // Exact first k inside each output's recorded chunk (as tg_gemm_dl): a
         // counting sort by chunk, then one output per thread at a time, every
@@ -490,32 +488,33 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
         int shift = 0;
         while (((nkt - 1) >> shift) >= Cfg::NB) ++shift;
         const int nb = ((nkt - 1) >> shift) + 1;
-        if (owner && tid < Cfg::NB) hist[tid] = 0;
+        const bool sorter = HALVES == 1 || half == 0;  // scans the buckets
+        if (sorter && tid < Cfg::NB) hist[tid] = 0;
         __syncthreads();
-        if (owner) {
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < ER; ++i) {
+            if (i >= ern) break;
 #pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    chs[trow(i) * BN + tcol(j)] = ch[i][j] < 0 ? NONE : uint16_t(ch[i][j]);
-                    if (ch[i][j] >= 0) atomicAdd(&hist[ch[i][j] >> shift], 1u);
-                }
+            for (int j = 0; j < TN; ++j) {
+                chs[erow(i) * BN + tcol(j)] = ch[i][j] < 0 ? NONE : uint16_t(ch[i][j]);
+                if (ch[i][j] >= 0) atomicAdd(&hist[ch[i][j] >> shift], 1u);
+            }
         }
         __syncthreads();
-        const int cnt = owner && tid < nb ? int(hist[tid]) : 0;
+        const int cnt = sorter && tid < nb ? int(hist[tid]) : 0;
         int total = 0;
         const int start = block_exclusive_scan(cnt, misc, total, tid);
-        if (owner && tid < nb) hist[tid] = uint32_t(start);
+        if (sorter && tid < nb) hist[tid] = uint32_t(start);
         if (HALVES > 1 && threadIdx.x == 0) *shared_total = total;
         __syncthreads();
         if constexpr (HALVES > 1) total = *shared_total;
-        if (owner) {
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < ER; ++i) {
+            if (i >= ern) break;
 #pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    if (ch[i][j] >= 0)
-                        list[atomicAdd(&hist[ch[i][j] >> shift], 1u)] = uint16_t(trow(i) * BN + tcol(j));
+            for (int j = 0; j < TN; ++j)
+                if (ch[i][j] >= 0)
+                    list[atomicAdd(&hist[ch[i][j] >> shift], 1u)] = uint16_t(erow(i) * BN + tcol(j));
         }
         __syncthreads();
         constexpr int NW = CL / 2;  // 16-byte vectors per window
@@ -557,28 +556,27 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
             chs[lid] = uint16_t(uint32_t(f) | neg);
         }
         __syncthreads();
-        if (owner) {
 #pragma unroll
-            for (int i = 0; i < TM; ++i) {
+        for (int i = 0; i < ER; ++i) {
+            if (i >= ern) break;
 #pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    if (ch[i][j] == -2) {  // redone below
-                        ch[i][j] = 0;
-                    } else if (ch[i][j] < 0) {  // the tropical zero was never beaten
-                        acc[i][j] = tzero<SR, T>();
-                        ch[i][j] = 0;
-                    } else {
-                        const int r = chs[trow(i) * BN + tcol(j)];
-                        ch[i][j] = ch[i][j] * CL + (r & 31);
-                        if constexpr (F64) {
-                            if (acc[i][j] == T(0)) acc[i][j] = (r & 32) ? -T(0) : T(0);
-                        }
+            for (int j = 0; j < TN; ++j) {
+                if (ch[i][j] == -2) {  // redone below
+                    ch[i][j] = 0;
+                } else if (ch[i][j] < 0) {  // the tropical zero was never beaten
+                    acc[i][j] = tzero<SR, T>();
+                    ch[i][j] = 0;
+                } else {
+                    const int r = chs[erow(i) * BN + tcol(j)];
+                    ch[i][j] = ch[i][j] * CL + (r & 31);
+                    if constexpr (F64) {
+                        if (acc[i][j] == T(0)) acc[i][j] = (r & 32) ? -T(0) : T(0);
                     }
                 }
-                store_row(i);
             }
-            if constexpr (F64) redo_outputs();
+            store_row(i);
         }
+        if constexpr (F64) redo_outputs();
     }
 }
 
