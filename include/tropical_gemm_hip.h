@@ -194,7 +194,9 @@ size_t tg_gemm_noalloc_bytes(tg_semiring semiring, tg_dtype dtype, tg_layout lay
  * The (strided batched) product when its outputs are few or narrow, by a
  * kernel of its own that needs no workspace and allocates nothing (fine under
  * graph capture): tiles of 4 x 16 up to 32 x 32 outputs whose K is split over
- * the lanes and waves of a workgroup.  *ran is 1 when the product was
+ * the lanes and waves of a workgroup; or, for i32 MaxPlus/MinPlus argmax at
+ * short K with few row tiles per item, the "kresg" kernel of tg_gemm_plan.
+ * *ran is 1 when the product was
  * launched; 0 when another kernel is the faster one for these sizes (or they
  * are empty): nothing was launched, and the caller goes on to one of the entry
  * points below or above, which keep their own kernels (tg_gemm_plan).  The
@@ -208,7 +210,7 @@ int tg_gemm_small(int device, tg_semiring semiring, tg_dtype dtype, tg_layout la
                   void* stream, int* ran);
 
 /* The launch tg_gemm_small would use ("16x16 waves 4": output tile and waves
- * per workgroup), "none" when it would leave the problem to the other entry
+ * per workgroup; "kresg"), "none" when it would leave the problem to the other entry
  * points, "invalid" for arguments the call would reject.  Strides 0 mean
  * dense single products.  Host logic only, as tg_gemm_plan; diagnostic. */
 const char* tg_gemm_small_plan(tg_semiring semiring, tg_dtype dtype, tg_layout layout,

@@ -32,8 +32,9 @@ def test_element_loads_edges(dt, m, n, k):
         # Up to 256 tiles, K from 256 runs in two (1024: four) slices, value-only in
         # four.
         cut = k >= 256
+        keys = dt == "i32" and sr != "maxmul" and k <= 160  # tg_gemm_kresg
         assert nat.gemm_plan(sr, dt, m, n, k, True) == (
-            "dl_elem_cl8" + (" slices 4" if k >= 1024 else " slices 2" if cut else ""))
+            "kresg" if keys else "dl_elem_cl8" + (" slices 4" if k >= 1024 else " slices 2" if cut else ""))
         assert nat.gemm_plan(sr, dt, m, n, k, False) == "dl_elem" + (" slices 4" if cut else "")
         # Ties across k, and winners in the last, partial window.
         lo, hi = (1, 50) if sr == "maxmul" else (-50, 50)
@@ -91,15 +92,16 @@ def test_element_loads_misaligned_batches(dt):
     """Sizes that are whole vectors, batch strides that are not."""
     from tropical_gemm import _native as nat
 
+    sr = "minplus" if dt == "f32" else "maxmul"  # i32 MinPlus: tg_gemm_kresg
     m, n, k = 320, 384, 160
     strides = (m * k + 1, k * n, m * n + 3)
-    assert nat.gemm_plan("minplus", dt, m, n, k, True, batch=3, strides=strides) == "dl_elem_cl8"
+    assert nat.gemm_plan(sr, dt, m, n, k, True, batch=3, strides=strides) == "dl_elem_cl8"
     rng = np.random.default_rng(12)
     items = [(tc.rng_matrix(rng, tc.NP_DTYPES[dt], (m, k), -1000, 1000),
               tc.rng_matrix(rng, tc.NP_DTYPES[dt], (k, n), -1000, 1000)) for _ in range(3)]
     print(f"[case] element loads misaligned batch {dt}", flush=True)
-    for (x, y), (c, am) in zip(items, _strided_batched("minplus", items, gap_a=1, gap_c=3)):
-        assert_exact(c, am, *oracle.gemm("minplus", x, y))
+    for (x, y), (c, am) in zip(items, _strided_batched(sr, items, gap_a=1, gap_c=3)):
+        assert_exact(c, am, *oracle.gemm(sr, x, y))
 
 
 def test_short_k_without_workspace_keeps_the_exact_mode():

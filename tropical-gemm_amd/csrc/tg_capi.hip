@@ -25,6 +25,7 @@
 #include "tg_gemm_kresw.hpp"
 #include "tg_gemm_shortk.hpp"
 #include "tg_kernels.hpp"
+#include "tg_kresg.hpp"
 #include "tg_small.hpp"
 
 namespace {
@@ -696,6 +697,15 @@ int launch_kresw(const Problem& p, int64_t tiles_n, hipStream_t st) {
     return TG_OK;
 }
 
+int run_gemm_kresg(int sr, const Problem& p, hipStream_t st) {
+    KernelTimer timer(st);
+    TG_HIP(tg::kresg_launch(
+        tg::KresgProblem{sr, static_cast<const int32_t*>(p.A), static_cast<const int32_t*>(p.B),
+                         static_cast<int32_t*>(p.C), p.IDX, p.batch, p.M, p.N, p.K, p.sA, p.sB, p.sC},
+        current_cu_count(), st));
+    return TG_OK;
+}
+
 template <int SR>
 int run_gemm_kresw(const Problem& p, hipStream_t st) {
     using Cfg = tg::KreswCfg;
@@ -805,7 +815,7 @@ constexpr int64_t kShortkArgmaxMaxK = 32;
 constexpr int64_t kShortkValueMaxK = 63;
 
 // The kernel a problem runs on.
-enum class Path { SHORTK, KRESW, KRES8, KRES, DL_88_32, DL_48_16, DL_48_VALUE, DL_44_8, DL_44_16, DL_44_32, DL_ELEM_8, DL_ELEM_16, DL_ELEM, DL64, DL64_VALUE, DL64S, DL64S_VALUE, TILES_EXACT, TILES_CHUNKED, TILES };
+enum class Path { SHORTK, KRESW, KRES8, KRES, KRESG, DL_88_32, DL_48_16, DL_48_VALUE, DL_44_8, DL_44_16, DL_44_32, DL_ELEM_8, DL_ELEM_16, DL_ELEM, DL64, DL64_VALUE, DL64S, DL64S_VALUE, TILES_EXACT, TILES_CHUNKED, TILES };
 
 struct Plan {
     Path path = Path::TILES;
@@ -821,6 +831,7 @@ bool uses_workspace(const Plan& pl, bool argmax) {
         case Path::KRESW:
         case Path::KRES8:
         case Path::KRES:
+        case Path::KRESG:
         case Path::DL_ELEM:
         case Path::TILES_EXACT:
         case Path::TILES: return false;
@@ -833,6 +844,32 @@ bool uses_workspace(const Plan& pl, bool argmax) {
     }
 }
 
+// True when tg_gemm_kresg is the kernel for an i32 MaxPlus/MinPlus argmax
+// problem that the kernels for aligned sizes (kresw, kres8, kres) leave.
+// Measured on MI355X (us, against the path it would take otherwise; in the key
+// range, then with wide operands):
+//   K <= 32, against the short-K kernel, which writes 256-column tiles: 100000
+//     x 64 x 12 18 / 44, x 128 x 16 25 / 53, x 256 x 24 43 / 76, 30000 x 200 x
+//     16 24 / 19, x 24 25 / 26; wide 262144 x 32 x 32 55 / 234, 50000 x 128 x
+//     20 27 / 36.
+//   K <= 160, against the generic exact mode and the direct-to-LDS kernels:
+//     300 x 300 x 36 10 / 15, 20000 x 48 x 48 11 / 19, 4096^2 x 100 80 / 193,
+//     200 x 20000 x 160 46 / 81; wide 20000 x 48 x 48 15 / 19, x 160 x 160 55 /
+//     66, 262144 x 160 x 160 537 / 585.
+//   beyond, 512 x 512 x 200 35 / 33, 20000 x 200 x 200 68 / 97, 4096 x 1024 x
+//     240 43 / 85; wide 4096 x 1024 x 240 72 / 90, but 20000 x 200 x 240 133 /
+//     105, whose wave tiles fill 1.2 rounds of the chip's 4096 waves: from
+//     three quarters of the last round up.
+bool takes_kresg(const Problem& p) {
+    if (!tg::kresg_fits(p.M, p.N, p.K) || p.M < 32) return false;
+    const int64_t tiles = tg::kresg_wave_tiles(p.M, p.N) * p.batch;
+    if (tiles < 64) return false;
+    if (p.K <= 32) return (p.N <= 64 && p.K >= 12) || (p.N <= 256 && p.K >= 20);
+    if (p.K <= 160) return true;
+    const int64_t rounds = (tiles + 4095) / 4096;
+    return 4 * tiles >= 3 * 4096 * rounds;
+}
+
 // Chooses the kernel.  ws_bytes limits split K (the partials live in the
 // workspace).
 template <int SR, typename T>
@@ -840,6 +877,11 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
     Plan pl;
     const bool argmax = p.IDX != nullptr;
     const bool exact = argmax && p.K <= kExactMaxK;
+    const bool kresg = std::is_same<T, int32_t>::value && SR != tg::SR_MAXMUL && argmax && takes_kresg(p);
+    if (kresg && p.K <= 32) {
+        pl.path = Path::KRESG;
+        return pl;
+    }
     if (p.K <= (argmax ? kShortkArgmaxMaxK : kShortkValueMaxK) &&
         tg::shortk_fits(p.M, p.N, p.K, p.sB, p.sC, p.B, p.C, p.IDX)) {
         pl.path = Path::SHORTK;
@@ -858,6 +900,10 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
         }
         if (argmax && tg::kres_fits(p.M, p.N, p.K, p.sA, p.sB, p.sC, p.A, p.B, p.C, p.IDX)) {
             pl.path = Path::KRES;
+            return pl;
+        }
+        if (kresg) {
+            pl.path = Path::KRESG;
             return pl;
         }
         // Partial tiles (M, N or K): short argmax problems take the generic
@@ -1038,6 +1084,10 @@ int run_gemm_typed(const Problem& p, void* ws, size_t ws_bytes, hipStream_t st) 
                     return run_gemm_kres8<SR>(p, st);
                 break;
             case Path::KRES: return run_gemm_kres<SR, T>(p, st);
+            case Path::KRESG:
+                if constexpr (std::is_same<T, int32_t>::value && SR != tg::SR_MAXMUL)
+                    return run_gemm_kresg(SR, p, st);
+                break;
             case Path::DL_88_32: return run_gemm_dl<SR, T, 8, 8, 32>(p, ws, 1, st);
             case Path::DL_48_16: return run_gemm_dl<SR, T, 4, 8, 16>(p, ws, 1, st);
             case Path::DL_48_VALUE: return run_gemm_dl<SR, T, 4, 8, 16>(p, ws, 1, st);  // CL unused
@@ -1158,6 +1208,7 @@ const char* path_name(Path path) {
         case Path::KRESW: return "kresw";
         case Path::KRES8: return "kres8";
         case Path::KRES: return "kres";
+        case Path::KRESG: return "kresg";
         case Path::DL_88_32: return "dl_8x8_cl32";
         case Path::DL_48_16: return "dl_4x8_cl16";
         case Path::DL_48_VALUE: return "dl_4x8";
@@ -1346,6 +1397,10 @@ tg::SmallProblem small_problem(tg_semiring sr, tg_dtype dt, const Problem& p) {
 //   direct-to-LDS with element loads (32-bit): f32 argmax 701^3 37 / 54, 734 x
 //     1071 x 3636 232 / 180, 1001^3 102 / 76; value-only 701^3 27 / 29, 734 x
 //     1071 x 3636 195 / 136 (i32 198 / 186); unsliced 1500^2 x 150 47 / 46.
+//   any short K (i32): 10000 x 20 x 20 8.6 / 6.8, 5000 x 32 x 32 6.6 / 6.9,
+//     5000 x 48 x 48 7.1 / 9.9, 10000 x 48 x 48 11.9 / 10.2, 5000 x 100 x 100
+//     14 / 17, 10000 x 100 x 100 21 / 18, 5000 x 160 x 160 20.4 / 20.4, 5000 x
+//     256 x 256 43 / 40.
 //   generic tiles, 32-bit (few tiles, or K <= 96): 42 x (452 x 92 x 52) f32
 //     argmax 23 / 28, 2001^2 x 60 45 / 41.
 //   f64: 700^3 argmax 79 / 111, value-only 54 / 78, 1024^3 207 / 149, 147 / 111;
@@ -1358,6 +1413,8 @@ int64_t small_output_limit(tg_dtype dt, const Plan& pl, const Problem& p) {
     constexpr int64_t k1 = int64_t(1) << 10;
     const bool argmax = p.IDX != nullptr;
     const int64_t narrow = p.M < p.N ? p.M : p.N;
+    if (pl.path == Path::KRESG)
+        return p.K <= 32 ? 192 * k1 : p.K <= 48 ? 384 * k1 : p.K <= 160 ? 768 * k1 : 1280 * k1;
     if (p.K <= 32) {
         if (p.N <= 64) return INT64_MAX;
         return !argmax ? 512 * k1 : dt == TG_F64 ? 128 * k1 : 256 * k1;
@@ -1393,15 +1450,25 @@ int64_t small_output_limit(tg_dtype dt, const Plan& pl, const Problem& p) {
     return 2048 * k1;
 }
 
-// True when tg_gemm_small takes the problem: `form` is its launch.
-bool choose_small(tg_semiring sr, tg_dtype dt, const Problem& p, tg::SmallForm* form) {
-    if (p.batch <= 0 || p.M <= 0 || p.N <= 0 || p.K <= 0) return false;
-    const Plan pl = plan_gemm(sr, dt, p, workspace_bytes_for(dt, p.batch, p.M, p.N, p.K,
-                                                             p.IDX != nullptr));
+// What tg_gemm_small runs: `form` is the few-output kernel's launch.
+enum class Small { NONE, FEW, KRESG };
+
+Small choose_small(tg_semiring sr, tg_dtype dt, const Problem& p, tg::SmallForm* form) {
+    if (p.batch <= 0 || p.M <= 0 || p.N <= 0 || p.K <= 0) return Small::NONE;
+    Plan pl = plan_gemm(sr, dt, p, workspace_bytes_for(dt, p.batch, p.M, p.N, p.K,
+                                                       p.IDX != nullptr));
+    // tg_gemm_kresw, one 16-wave workgroup per CU and one batch item after the
+    // other, while an item's wave tiles do not give each of the chip's waves
+    // more than one (us, kresw / kresg: 4096 x 1024 x 128 36 / 25, 32768 x 128 x
+    // 64 22 / 14, 8 x (4096 x 128 x 128) 251 / 28; 16384 x 512 x 128 40 / 45).
+    const bool few_wave_tiles = pl.path == Path::KRESW && takes_kresg(p) &&
+                                tg::kresg_wave_tiles(p.M, p.N) <= 4096;
+    if (few_wave_tiles) pl.path = Path::KRESG;
     // In floating point: batch * M * N of a caller's sizes may pass 2^63.
-    if (double(p.batch) * double(p.M) * double(p.N) >= double(small_output_limit(dt, pl, p)))
-        return false;
-    return tg::small_form(small_problem(sr, dt, p), form);
+    if (double(p.batch) * double(p.M) * double(p.N) < double(small_output_limit(dt, pl, p)) &&
+        tg::small_form(small_problem(sr, dt, p), form))
+        return Small::FEW;
+    return few_wave_tiles ? Small::KRESG : Small::NONE;
 }
 
 // ----------------------------------------------------------------------------
@@ -1874,12 +1941,18 @@ int tg_gemm_small(int device, tg_semiring semiring, tg_dtype dtype, tg_layout la
     const Problem p = make_problem(layout, A, B, C, argmax, batch, m, n, k, stride_a, stride_b,
                                    stride_c, true);
     tg::SmallForm form;
-    if (!choose_small(semiring, dtype, p, &form)) return TG_OK;
+    const Small kernel = choose_small(semiring, dtype, p, &form);
+    if (kernel == Small::NONE) return TG_OK;
     rc = select_device(device);
     if (rc != TG_OK) return rc;
     hipStream_t st = as_stream(stream);
-    KernelTimer timer(st);
-    TG_HIP(tg::small_launch(small_problem(semiring, dtype, p), form, st));
+    if (kernel == Small::KRESG) {
+        rc = run_gemm_kresg(semiring == TG_MAXPLUS ? tg::SR_MAXPLUS : tg::SR_MINPLUS, p, st);
+        if (rc != TG_OK) return rc;
+    } else {
+        KernelTimer timer(st);
+        TG_HIP(tg::small_launch(small_problem(semiring, dtype, p), form, st));
+    }
     *ran = 1;
     return TG_OK;
 }
@@ -1896,7 +1969,11 @@ const char* tg_gemm_small_plan(tg_semiring semiring, tg_dtype dtype, tg_layout l
     const Problem p = make_problem(layout, A, B, const_cast<void*>(C), const_cast<int32_t*>(argmax),
                                    batch, m, n, k, stride_a, stride_b, stride_c, strided);
     tg::SmallForm f;
-    if (!choose_small(semiring, dtype, p, &f)) return "none";
+    switch (choose_small(semiring, dtype, p, &f)) {
+        case Small::NONE: return "none";
+        case Small::KRESG: return "kresg";
+        case Small::FEW: break;
+    }
     name = std::to_string(4 * f.lr) + "x" + std::to_string(4 * f.lc) + " waves " +
            std::to_string(f.waves);
     return name.c_str();
