@@ -77,19 +77,19 @@ KERNEL_NAMES = {
     "M1": "tg_gemm_shortk<MaxPlus, f32, argmax> (32x256 tiles, per-product index)",
     "F1": "tg_gemm_dl64<MaxPlus> (f64, 64x128 tiles, argmax)",
     "F2": "tg_gemm_dl64<MaxPlus, value-only> (f64, 64x128 tiles)",
-    "I1": "tg_gemm_tiles<MaxPlus, i64, chunked argmax, 16-k chunks> (64x64 tiles)",
-    "I2": "tg_gemm_tiles<MaxPlus, i64, value-only> (64x64 tiles)",
+    "I1": "tg_gemm_dl64s<MaxPlus, i64, argmax> (64x64 tiles)",
+    "I2": "tg_gemm_dl64s<MaxPlus, i64, value-only> (64x64 tiles, two K slices)",
 }
 # HBM bytes per launch of the dominant kernel from rocprofv3 --pmc FETCH_SIZE
 # and WRITE_SIZE, scaled by the same counters on a copy kernel of known size
 # (profiles/tg_gemm_dl_maxplus_f32_4096_argmax.md, profiles/tg_gemm_kresw_*.md,
 # profiles/tg_gemm_shortk_*.md, profiles/hbm_traffic_c2_c3_e1.md,
 # profiles/tg_gemm_dl_split_*.md, profiles/tg_gemm_dl64_*.md,
-# profiles/tg_gemm_tiles_maxplus_i64_4096.md).  E1: per GEMM launch.
+# profiles/tg_gemm_dl64s_maxplus_i64_4096.md).  E1: per GEMM launch.
 
 TRAFFIC = {"P": 1.924e9, "C5": 1.924e9, "C4": 0.418e9, "M1": 1.108e9, "C1": 0.034e9,
            "C2": 1.771e9, "C3": 0.704e9, "F1": 3.439e9, "F2": 2.266e9, "E1": 0.1177e9,
-           "I1": 4.881e9, "I2": 3.356e9}
+           "I1": 4.452e9, "I2": 3.346e9}
 
 
 def cpu_model() -> str:
