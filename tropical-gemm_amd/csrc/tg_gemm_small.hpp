@@ -82,8 +82,8 @@ __device__ __forceinline__ double join_raw_f64(double x, double y) {
 // the four columns of a lane past the right edge shift left into the matrix
 // (columns that another lane owns: computed twice, stored once).
 // grid = (tiles_m * tiles_n, 1, batch), block = 64 * W, W <= MAX_WAVES,
-// LDS = SmallCfg::lds_bytes(W, ARGMAX).  M * K and K * N below 2^28 elements
-// (32-bit byte offsets).
+// LDS = SmallCfg::lds_bytes(W, ARGMAX).  M * K and K * N below 2^31 elements
+// (32-bit element offsets).
 template <int SR, typename T, bool ARGMAX, int LR, int LC, bool NCLAMP>
 __global__ __launch_bounds__(64 * small_max_waves<T>()) void tg_gemm_small(
     const T* __restrict__ A, const T* __restrict__ B, T* __restrict__ C, int32_t* __restrict__ IDX,
