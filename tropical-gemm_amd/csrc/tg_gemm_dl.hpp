@@ -20,6 +20,7 @@
 
 #include <utility>
 
+#include "tg_elem_rows.hpp"
 #include "tg_kernels.hpp"
 
 namespace tg {
@@ -443,12 +444,13 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
             lds_load4(ab + off, adst + ins * 64);
         }
         const int ins0 = wave * NBI * 4;
-        const unsigned char* bb = reinterpret_cast<const unsigned char*>(B + (t * BK + ins0 / EPR) * N);
+        const int first = elem_first_row(ins0 / EPR, left);
+        const unsigned char* bb = reinterpret_cast<const unsigned char*>(B + (t * BK + first) * N);
 #pragma unroll
         for (int q = 0; q < NBI * 4; ++q) {
             const int64_t gc = col0 + q % EPR * 64 + lane;
             lds_load4(bb + uint32_t((gc < N ? gc : N - 1) * 4), bdst + (ins0 + q) * 64);
-            if (q % EPR == EPR - 1 && (ins0 + q) / EPR + 1 < left) bb += N * 4;
+            if (q % EPR == EPR - 1 && elem_steps((ins0 + q) / EPR, left)) bb += N * 4;
         }
     };
     auto b_base = [&](int q, int64_t k0) {

@@ -38,6 +38,7 @@
 // tg_gemm_dl64; NaN for f64 by operand classes, as there (clsA / clsB).
 #pragma once
 
+#include "tg_elem_rows.hpp"
 #include "tg_gemm_dl64.hpp"
 
 namespace tg {
@@ -177,8 +178,7 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
         uint32_t k8 = uint32_t(K) * 8, n8 = uint32_t(N) * 8;
         if constexpr (ELEM) {
             asm volatile("" : "+s"(k8), "+s"(n8));
-            const int first = wave * (BK / 4);  // the wave's k rows of B
-            bb += uint64_t(first < left ? first : left - 1) * n8;
+            bb += uint64_t(elem_first_row(wave * (BK / 4), left)) * n8;  // the wave's k rows of B
         }
 #pragma unroll
         for (int q = 0; q < NL; ++q) {
@@ -193,7 +193,7 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
                 const unsigned char* row = ab + (r < max_row ? r : max_row) * k8;
                 lds_load4(row + ((r < max_row ? rowK : 0u) + uint32_t(byte)), adst + ins * IB);
                 lds_load4(bb + offB[q % 2], bdst + ins * IB);
-                if (q % 2 == 1 && ins / 2 + 1 < left) bb += n8;
+                if (q % 2 == 1 && elem_steps(ins / 2, left)) bb += n8;
             } else {
                 uint32_t oa = offA[q], ob = offB[0];
                 if (last) {
