@@ -132,8 +132,8 @@ def test_f64_configs_full_size(name, with_argmax, plan):
         np.testing.assert_array_equal(am.cpu().numpy()[rows], am_ref.astype(np.int32))
 
 
-@pytest.mark.parametrize("name,with_argmax,plan", [("I1", True, "tiles_chunked"),
-                                                   ("I2", False, "tiles")])
+@pytest.mark.parametrize("name,with_argmax,plan", [("I1", True, "dl64s_4x4_cl16"),
+                                                   ("I2", False, "dl64s_4x4")])
 def test_i64_configs_full_size(name, with_argmax, plan):
     """I1 / I2 (MaxPlus i64 4096^3, entries in [-10^9, 10^9]) at full size:
     argmax consistency on every output (I1), the oracle on sampled rows

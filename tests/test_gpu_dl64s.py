@@ -12,8 +12,7 @@ from tests.test_gpu_parity import _strided_batched, assert_exact, gpu_gemm
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
-PLAN = {("f64", True): "dl64s_4x4_cl16", ("f64", False): "dl64s_4x4",
-        ("i64", True): "tiles_chunked", ("i64", False): "tiles"}
+PLAN = {True: "dl64s_4x4_cl16", False: "dl64s_4x4"}
 
 # Up to 256 tiles K runs in three (argmax) or four slices, above in one or two.
 # (m, n, k): a last k-tile of 1, 2, 15 and 16 k, 17 and 18 k-tiles (slices of
@@ -49,7 +48,7 @@ def test_dl64s_edges(dt, m, n, k):
         a, b = _data(sr, tc.NP_DTYPES[dt], m, n, k)
         c_ref, am_ref = oracle.gemm(sr, a, b)
         for with_argmax in (True, False):
-            assert nat.gemm_plan(sr, dt, m, n, k, with_argmax) == PLAN[dt, with_argmax]
+            assert nat.gemm_plan(sr, dt, m, n, k, with_argmax) == PLAN[with_argmax]
             print(f"[case] dl64s {sr} {dt} {m}x{n}x{k} argmax={with_argmax}", flush=True)
             c, am = gpu_gemm(sr, a, b, with_argmax)
             assert_exact(c, am, c_ref, am_ref if with_argmax else None)
@@ -92,6 +91,6 @@ def test_dl64s_wrapping_zeros_and_batches(dt):
 def test_i64_without_workspace_keeps_the_exact_mode():
     from tropical_gemm import _native as nat
 
-    assert nat.gemm_plan("maxplus", "i64", 512, 40000, 300, True) == "tiles_chunked"
+    assert nat.gemm_plan("maxplus", "i64", 512, 40000, 300, True) == "dl64s_4x4_cl16"
     assert nat.gemm_plan("maxplus", "i64", 512, 40000, 300, True,
                          workspace_bytes=64 << 20) == "tiles_exact"

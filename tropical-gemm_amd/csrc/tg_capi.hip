@@ -815,7 +815,7 @@ constexpr int64_t kShortkArgmaxMaxK = 32;
 constexpr int64_t kShortkValueMaxK = 63;
 
 // The kernel a problem runs on.
-enum class Path { SHORTK, KRESW, KRES8, KRES, KRESG, DL_88_32, DL_48_16, DL_48_VALUE, DL_44_8, DL_44_16, DL_44_32, DL_ELEM_8, DL_ELEM_16, DL_ELEM, DL64, DL64_VALUE, DL64S, DL64S_VALUE, TILES_EXACT, TILES_CHUNKED, TILES };
+enum class Path { SHORTK, KRESW, KRES8, KRES, KRESG, DL_88_32, DL_48_16, DL_48_VALUE, DL_44_8, DL_44_16, DL_44_32, DL_ELEM_8, DL_ELEM_16, DL_ELEM, DL64, DL64_VALUE, DL64S, DL64S_VALUE, DL64S_I64, DL64S_I64_VALUE, TILES_EXACT, TILES_CHUNKED, TILES };
 
 struct Plan {
     Path path = Path::TILES;
@@ -833,13 +833,15 @@ bool uses_workspace(const Plan& pl, bool argmax) {
         case Path::KRES:
         case Path::KRESG:
         case Path::DL_ELEM:
+        case Path::DL64S_I64_VALUE:
         case Path::TILES_EXACT:
         case Path::TILES: return false;
         case Path::TILES_CHUNKED:
         case Path::DL64:
         case Path::DL64_VALUE:
         case Path::DL64S:
-        case Path::DL64S_VALUE: return true;
+        case Path::DL64S_VALUE:
+        case Path::DL64S_I64: return true;
         default: return argmax || pl.splits > 1;
     }
 }
@@ -1047,12 +1049,16 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
             }
         }
     }
+    // i64: the chunked and the value-only tiles are tg_gemm_dl64s; the
+    // register-staged kernel keeps sizes it does not fit and value-only K below
+    // 64 (2048^2 x 80: 52 us both).
+    const bool i64_dl = std::is_same<T, int64_t>::value && tg::dl64s_fits(p.M, p.N, p.K);
     if (!argmax)
-        pl.path = Path::TILES;
+        pl.path = i64_dl && p.K >= 64 ? Path::DL64S_I64_VALUE : Path::TILES;
     else if (exact || (p.K <= exact_tiles_max_k<T>() && !chunked_i64<T>(p, ws_bytes)))
         pl.path = Path::TILES_EXACT;
     else
-        pl.path = Path::TILES_CHUNKED;
+        pl.path = i64_dl ? Path::DL64S_I64 : Path::TILES_CHUNKED;
     return pl;
 }
 
@@ -1066,11 +1072,7 @@ int run_gemm_typed(const Problem& p, void* ws, size_t ws_bytes, hipStream_t st) 
             return run_gemm_dl64s<SR, double>(p, ws, st);
     }
     if constexpr (std::is_same<T, int64_t>::value) {
-        // The chunked and the value-only tiles of i64 are tg_gemm_dl64s; the
-        // register-staged kernel keeps sizes it does not fit and value-only
-        // K below 64 (2048^2 x 80: 52 us both).
-        if ((pl.path == Path::TILES_CHUNKED || (pl.path == Path::TILES && p.K >= 64)) &&
-            tg::dl64s_fits(p.M, p.N, p.K))
+        if (pl.path == Path::DL64S_I64 || pl.path == Path::DL64S_I64_VALUE)
             return run_gemm_dl64s<SR, int64_t>(p, ws, st);
     }
     if constexpr (sizeof(T) == 4) {
@@ -1220,8 +1222,10 @@ const char* path_name(Path path) {
         case Path::DL_ELEM: return "dl_elem";
         case Path::DL64: return "dl64_4x8_cl16";
         case Path::DL64_VALUE: return "dl64_4x8";
-        case Path::DL64S: return "dl64s_4x4_cl16";
-        case Path::DL64S_VALUE: return "dl64s_4x4";
+        case Path::DL64S:
+        case Path::DL64S_I64: return "dl64s_4x4_cl16";
+        case Path::DL64S_VALUE:
+        case Path::DL64S_I64_VALUE: return "dl64s_4x4";
         case Path::TILES_EXACT: return "tiles_exact";
         case Path::TILES_CHUNKED: return "tiles_chunked";
         case Path::TILES: return "tiles";
@@ -1355,7 +1359,7 @@ int gemm_impl(int device, tg_semiring sr, tg_dtype dt, tg_layout layout, const v
             const Plan pl = plan_gemm(sr, dt, p, ws_bytes);
             if (!uses_workspace(pl, with_argmax)) {
                 ws_bytes = 0;
-            } else if ((pl.path == Path::DL_ELEM_8 || pl.path == Path::TILES_CHUNKED ||
+            } else if ((pl.path == Path::DL_ELEM_8 || pl.path == Path::DL64S_I64 ||
                         pl.path == Path::DL64S || pl.path == Path::DL64S_VALUE) &&
                        !uses_workspace(plan_gemm(sr, dt, p, 0), with_argmax)) {
                 // Under capture a product that these paths took from a kernel
@@ -1429,6 +1433,8 @@ int64_t small_output_limit(tg_dtype dt, const Plan& pl, const Problem& p) {
         case Path::DL64_VALUE: return 2048 * k1;
         case Path::DL64S:
         case Path::DL64S_VALUE: return narrow <= 32 ? 2048 * k1 : 768 * k1;
+        case Path::DL64S_I64:
+        case Path::DL64S_I64_VALUE:
         case Path::TILES_EXACT:
         case Path::TILES_CHUNKED:
         case Path::TILES: break;
