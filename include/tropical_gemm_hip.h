@@ -173,7 +173,10 @@ int tg_gemm_ws(int device, tg_semiring semiring, tg_dtype dtype, tg_layout layou
  * k x max(m, n) elements above it on the chunked-argmax paths) is rejected
  * with TG_ERR_INVALID_ARGUMENT before any device work.  Every call on one
  * device shares that device's array, so calls that overlap on one device
- * (other streams, other host threads) race; serialise them.  The kernels
+ * (other streams, other host threads) race; serialise them.  Calls whose
+ * tg_gemm_noalloc_bytes is 0 leave it alone and may overlap; a product that a
+ * kernel without a workspace can run takes that one here, also where tg_gemm
+ * has a faster one that needs it.  The kernels
  * write every scratch byte they read, so nothing needs clearing between
  * calls.  Same arguments, results and errors as tg_gemm otherwise. */
 #define TG_NOALLOC_SCRATCH_BYTES ((size_t)64 << 20)

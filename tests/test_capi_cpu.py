@@ -210,3 +210,26 @@ def test_noalloc_bytes_of_other_paths():
     assert _noalloc_bytes("maxplus", "i32", 262144, 128, 128, True) == 0
     assert _noalloc_bytes("maxplus", "f32", 0, 4, 4, True) == 0
     assert _noalloc_bytes("maxplus", "f32", -1, 4, 4, True) == 2**64 - 1
+
+
+@pytest.mark.parametrize("dt,m,n,k,argmax", [
+    ("f32", 1000, 1001, 300, True),   # element loads in tg_gemm; the exact tiles without a workspace
+    ("i32", 1000, 1001, 300, True),
+    ("f64", 1500, 1500, 512, True),   # 64 x 64 tiles with operand classes (and B^T)
+    ("f64", 1000, 1000, 400, False),
+    ("i64", 1000, 1000, 1000, True),  # 64 x 64 tiles with B^T
+])
+def test_noalloc_leaves_the_scratch_to_products_that_need_it(dt, m, n, k, argmax):
+    """Calls that share no scratch may overlap on other streams and threads:
+    a product that can run without one does."""
+    assert nat.gemm_plan("maxmul", dt, m, n, k, argmax).startswith(("dl_elem", "dl64s"))
+    assert _noalloc_bytes("maxmul", dt, m, n, k, argmax) == 0
+
+
+def test_noalloc_scratch_where_no_kernel_is_without():
+    # Argmax beyond the exact tiles' range, and value-only f64 that the 64 x 128
+    # tiles (operand classes) can run.
+    assert _noalloc_bytes("maxplus", "f32", 1000, 1001, 400, True) >= 1001 * 400 * 4
+    assert _noalloc_bytes("maxplus", "i64", 500, 500, 2100, True) >= 500 * 2100 * 8
+    assert _noalloc_bytes("maxplus", "f64", 1000, 1000, 520, True) >= 1000 * 520 * 8
+    assert _noalloc_bytes("maxplus", "f64", 1024, 2048, 512, False) == (1024 + 2048) * 4

@@ -846,6 +846,12 @@ bool uses_workspace(const Plan& pl, bool argmax) {
     }
 }
 
+// 64 x 128 tiles of a problem (tg_gemm_dl64).
+int64_t dl64_tiles(const Problem& p) {
+    return ((p.M + tg::Dl64Cfg::BM - 1) / tg::Dl64Cfg::BM) *
+           ((p.N + tg::Dl64Cfg::BN - 1) / tg::Dl64Cfg::BN) * p.batch;
+}
+
 // True when tg_gemm_kresg is the kernel for an i32 MaxPlus/MinPlus argmax
 // problem that the kernels for aligned sizes (kresw, kres8, kres) leave.
 // Measured on MI355X (us, against the path it would take otherwise; in the key
@@ -1034,8 +1040,7 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
         // 518 / 1053, 3001^2 x 300 376 / 459, 3000 x 2000 x 256 221 / 250;
         // value-only 1536^2 x 768 200 / 263, 1024^3 111 / 203, 3001^2 x 300
         // 249 / 323.
-        const int64_t tiles = ((p.M + tg::Dl64Cfg::BM - 1) / tg::Dl64Cfg::BM) *
-                              ((p.N + tg::Dl64Cfg::BN - 1) / tg::Dl64Cfg::BN) * p.batch;
+        const int64_t tiles = dl64_tiles(p);
         const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
         if (p.K >= 256 && dl64_ws_bytes(p.batch, p.M, p.N, p.K, argmax) <= ws_bytes) {
             if (tiles >= 512 && (!argmax || p.K > exact_tiles_max_k<T>()) &&
@@ -1322,6 +1327,26 @@ Problem make_problem(tg_layout layout, const void* A, const void* B, void* C, in
     return p;
 }
 
+// True when pl's workspace is a gain and not a need: without one the product
+// runs on the generic tiles, which read none.  Callers that share one workspace
+// (tg_gemm_noalloc) or would have to allocate it inside a capture use those.
+// Value-only f64 that the 64 x 128 tiles can run needs it either way (operand
+// classes).
+bool workspace_optional(tg_semiring sr, tg_dtype dt, const Problem& p, const Plan& pl) {
+    switch (pl.path) {
+        case Path::DL_ELEM_8:
+        case Path::DL64S:
+        case Path::DL64S_I64: break;
+        case Path::DL64S_VALUE:
+            if (dl64_tiles(p) >= 256 &&
+                tg::dl64_fits(p.M, p.N, p.K, p.sA, p.sB, p.sC, p.A, p.B, p.C, p.IDX))
+                return false;
+            break;
+        default: return false;
+    }
+    return !uses_workspace(plan_gemm(sr, dt, p, 0), p.IDX != nullptr);
+}
+
 int gemm_impl(int device, tg_semiring sr, tg_dtype dt, tg_layout layout, const void* A,
               const void* B, void* C, int32_t* argmax, int64_t batch, int64_t m, int64_t n,
               int64_t k, int64_t sa, int64_t sb, int64_t sc, bool strided, void* ws,
@@ -1359,11 +1384,8 @@ int gemm_impl(int device, tg_semiring sr, tg_dtype dt, tg_layout layout, const v
             const Plan pl = plan_gemm(sr, dt, p, ws_bytes);
             if (!uses_workspace(pl, with_argmax)) {
                 ws_bytes = 0;
-            } else if ((pl.path == Path::DL_ELEM_8 || pl.path == Path::DL64S_I64 ||
-                        pl.path == Path::DL64S || pl.path == Path::DL64S_VALUE) &&
-                       !uses_workspace(plan_gemm(sr, dt, p, 0), with_argmax)) {
-                // Under capture a product that these paths took from a kernel
-                // without a workspace goes back to it: no allocation nodes.
+            } else if (workspace_optional(sr, dt, p, pl)) {
+                // Under capture such a product runs without: no allocation nodes.
                 hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
                 if (hipStreamIsCapturing(st, &cap) != hipSuccess) (void)hipGetLastError();
                 if (cap != hipStreamCaptureStatusNone) ws_bytes = 0;
@@ -1513,9 +1535,20 @@ int scratch_address(int device, void** out) {
     return TG_OK;
 }
 
-// Scratch bytes the planned path reads (0 when it reads none).  The plan is
-// made with kScratchBytes as the workspace, so split K is only chosen when
-// its partials fit; B^T staging alone may still exceed it.
+// Plan of a tg_gemm_noalloc call, with kScratchBytes as the workspace, so
+// split K is only chosen when its partials fit.  Every call shares the scratch,
+// so a product that can run without it does (*ws_bytes is 0 then): such calls
+// may overlap.
+Plan scratch_plan(tg_semiring sr, tg_dtype dt, const Problem& p, size_t* ws_bytes) {
+    *ws_bytes = kScratchBytes;
+    const Plan pl = plan_gemm(sr, dt, p, kScratchBytes);
+    if (!workspace_optional(sr, dt, p, pl)) return pl;
+    *ws_bytes = 0;
+    return plan_gemm(sr, dt, p, 0);
+}
+
+// Scratch bytes the planned path reads (0 when it reads none).  B^T staging
+// alone may exceed the scratch.
 size_t scratch_need(tg_dtype dt, const Problem& p, const Plan& pl) {
     const bool argmax = p.IDX != nullptr;
     if (!uses_workspace(pl, argmax)) return 0;
@@ -1994,7 +2027,8 @@ int tg_gemm_noalloc(int device, tg_semiring semiring, tg_dtype dtype, tg_layout 
     // Host-only planning first, so an oversized problem is rejected before
     // any device work.
     const bool empty = m == 0 || n == 0;
-    const Plan pl = empty ? Plan{} : plan_gemm(semiring, dtype, p, kScratchBytes);
+    size_t ws_bytes = 0;
+    const Plan pl = empty ? Plan{} : scratch_plan(semiring, dtype, p, &ws_bytes);
     const size_t need = empty ? 0 : scratch_need(dtype, p, pl);
     if (need > kScratchBytes)
         return fail(TG_ERR_INVALID_ARGUMENT,
@@ -2007,7 +2041,7 @@ int tg_gemm_noalloc(int device, tg_semiring semiring, tg_dtype dtype, tg_layout 
     void* ws = nullptr;
     rc = scratch_address(device, &ws);
     if (rc != TG_OK) return rc;
-    return run_gemm(semiring, dtype, p, ws, kScratchBytes, as_stream(stream));
+    return run_gemm(semiring, dtype, p, ws, ws_bytes, as_stream(stream));
 }
 
 size_t tg_gemm_noalloc_bytes(tg_semiring semiring, tg_dtype dtype, tg_layout layout,
@@ -2018,7 +2052,9 @@ size_t tg_gemm_noalloc_bytes(tg_semiring semiring, tg_dtype dtype, tg_layout lay
     if (m == 0 || n == 0) return 0;
     const Problem p = make_problem(layout, A, B, const_cast<void*>(C), const_cast<int32_t*>(argmax),
                                    1, m, n, k, 0, 0, 0, false);
-    return scratch_need(dtype, p, plan_gemm(semiring, dtype, p, kScratchBytes));
+    size_t ws_bytes = 0;
+    const Plan pl = scratch_plan(semiring, dtype, p, &ws_bytes);
+    return scratch_need(dtype, p, pl);
 }
 
 size_t tg_gemm_workspace_size(tg_dtype dtype, int64_t batch, int64_t m, int64_t n, int64_t k,
