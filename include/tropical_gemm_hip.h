@@ -132,7 +132,7 @@ size_t tg_gemm_workspace_size(tg_dtype dtype, int64_t batch, int64_t m, int64_t 
                               int with_argmax);
 
 /* Name of the kernel path tg_gemm_ws would run for this problem with a
- * workspace of workspace_bytes (tg_gemm passes tg_gemm_workspace_size), e.g.
+ * workspace of workspace_bytes (tg_gemm has tg_gemm_alloc_bytes), e.g.
  * "dl_4x8_cl16", "shortk", "tiles_exact", "dl_4x4_cl32 split 4" (K in four
  * launches merged afterwards) or "dl_4x4_cl8 slices 4" (four K slices in one
  * workgroup per tile); "invalid" for arguments the call would reject, "none"
@@ -145,6 +145,17 @@ const char* tg_gemm_plan(tg_semiring semiring, tg_dtype dtype, tg_layout layout,
                          int64_t batch, int64_t m, int64_t n, int64_t k,
                          int64_t stride_a, int64_t stride_b, int64_t stride_c,
                          size_t workspace_bytes);
+
+/* Bytes of workspace tg_gemm (strides 0) or tg_gemm_strided_batched allocates
+ * and frees on the stream for this problem, outside a capture: 0 when its
+ * kernel reads none, or when a kernel that reads none is as fast as one that
+ * does with its allocation.  (size_t)-1 for arguments the call would reject.
+ * Host logic only, as tg_gemm_plan; diagnostic, with no counterpart in the
+ * reference. */
+size_t tg_gemm_alloc_bytes(tg_semiring semiring, tg_dtype dtype, tg_layout layout,
+                           const void* A, const void* B, const void* C, const int32_t* argmax,
+                           int64_t batch, int64_t m, int64_t n, int64_t k,
+                           int64_t stride_a, int64_t stride_b, int64_t stride_c);
 
 /* Launch geometry the backward entry points would use for a gradient
  * (want_a: 1 for grad A, 0 for grad B), e.g. "rows lds waves=2 lds=32768

@@ -233,3 +233,24 @@ def test_noalloc_scratch_where_no_kernel_is_without():
     assert _noalloc_bytes("maxplus", "i64", 500, 500, 2100, True) >= 500 * 2100 * 8
     assert _noalloc_bytes("maxplus", "f64", 1000, 1000, 520, True) >= 1000 * 520 * 8
     assert _noalloc_bytes("maxplus", "f64", 1024, 2048, 512, False) == (1024 + 2048) * 4
+
+
+@pytest.mark.parametrize("dt,batch,m,n,k,argmax,allocates", [
+    # Tiles without a workspace, where one would have to be allocated per call.
+    ("f32", 16, 64, 1025, 97, True, False), ("f32", 16, 64, 1025, 200, True, True),
+    ("f32", 1, 50000, 50, 384, True, False), ("f32", 1, 1000, 1001, 97, True, True),
+    ("f64", 1, 1500, 1500, 300, True, False), ("f64", 1, 1500, 1500, 512, True, True),
+    ("f64", 128, 128, 128, 512, True, False), ("f64", 1, 1000, 1000, 512, False, True),
+    ("i64", 1, 1500, 1500, 188, True, False), ("i64", 1, 1500, 1500, 300, True, True),
+    ("i64", 256, 64, 64, 1000, True, False), ("i64", 1, 1000, 1000, 1000, True, True),
+    # Kernels that have to have one, and one that never does.
+    ("f32", 1, 4096, 4096, 4096, True, True), ("f64", 4, 64, 64, 640, True, True),
+    ("f32", 1, 4096, 4096, 4096, False, False),
+])
+def test_tg_gemm_allocates_a_workspace_where_it_pays(dt, batch, m, n, k, argmax, allocates):
+    lib = nat.load()
+    got = lib.tg_gemm_alloc_bytes(nat.SEMIRING["maxmul"], nat.DTYPE[dt], nat.LAYOUT["row"], 256,
+                                  256, 256, 256 if argmax else None, batch, m, n, k, m * k, k * n,
+                                  m * n)
+    full = lib.tg_gemm_workspace_size(nat.DTYPE[dt], batch, m, n, k, int(argmax))
+    assert got == (full if allocates else 0)

@@ -1347,6 +1347,38 @@ bool workspace_optional(tg_semiring sr, tg_dtype dt, const Problem& p, const Pla
     return !uses_workspace(plan_gemm(sr, dt, p, 0), p.IDX != nullptr);
 }
 
+// Whether an optional workspace of this size pays when the call itself has to
+// allocate and free it.  Between synchronisations the stream's pool keeps up to
+// 2 MB; beyond that a call that is waited for pays about 25 us and 2.5 us per MB
+// (MI355X), against what the path gains.  us, with the allocation / without a
+// workspace: f32 argmax 16 x (64 x 1025 x 97) 63 / 49, x 200 79 / 93, 50000 x 50
+// x 384 285 / 176, 1000 x 1001 x 97 (0.4 MB) 37 / 48; f64 argmax 1500^2 x 300 164
+// / 152, x 512 216 / 254, 128 x (128 x 128 x 512) 288 / 178; i64 argmax 1500^2 x
+// 188 159 / 150, x 300 209 / 235, 1000^3 223 / 256, 256 x (64 x 64 x 1000) 316 /
+// 257.
+bool allocation_pays(tg_dtype dt, const Problem& p, size_t bytes) {
+    constexpr size_t kMB = size_t(1) << 20;
+    if (bytes <= 2 * kMB || p.IDX == nullptr) return true;
+    const int64_t narrow = p.M < p.N ? p.M : p.N;
+    const double products = double(p.batch) * double(p.M) * double(p.N) * double(p.K);
+    if (dt == TG_F64) return narrow >= 256 && products >= 8e8;
+    if (dt == TG_I64) return narrow >= 256 && (p.K >= 800 || products >= 5.5e8);
+    return p.K >= 192 ? bytes <= 64 * kMB || narrow >= 128 : narrow >= 512;
+}
+
+// Bytes that tg_gemm allocates for the call: the full workspace, for the
+// kernels that read it.  *optional: the product can run without.
+size_t own_workspace(tg_semiring sr, tg_dtype dt, const Problem& p, bool* optional) {
+    *optional = false;
+    const bool argmax = p.IDX != nullptr;
+    const size_t bytes = workspace_bytes_for(dt, p.batch, p.M, p.N, p.K, argmax);
+    if (bytes == 0) return 0;
+    const Plan pl = plan_gemm(sr, dt, p, bytes);
+    if (!uses_workspace(pl, argmax)) return 0;
+    *optional = workspace_optional(sr, dt, p, pl);
+    return *optional && !allocation_pays(dt, p, bytes) ? 0 : bytes;
+}
+
 int gemm_impl(int device, tg_semiring sr, tg_dtype dt, tg_layout layout, const void* A,
               const void* B, void* C, int32_t* argmax, int64_t batch, int64_t m, int64_t n,
               int64_t k, int64_t sa, int64_t sb, int64_t sc, bool strided, void* ws,
@@ -1378,18 +1410,13 @@ int gemm_impl(int device, tg_semiring sr, tg_dtype dt, tg_layout layout, const v
     void* work = ws;
     bool own = false;
     if (!ws_given) {
-        // Allocate the full workspace only for the kernels that read it.
-        ws_bytes = workspace_bytes_for(dt, batch, m, n, k, with_argmax);
-        if (ws_bytes > 0) {
-            const Plan pl = plan_gemm(sr, dt, p, ws_bytes);
-            if (!uses_workspace(pl, with_argmax)) {
-                ws_bytes = 0;
-            } else if (workspace_optional(sr, dt, p, pl)) {
-                // Under capture such a product runs without: no allocation nodes.
-                hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-                if (hipStreamIsCapturing(st, &cap) != hipSuccess) (void)hipGetLastError();
-                if (cap != hipStreamCaptureStatusNone) ws_bytes = 0;
-            }
+        bool optional;
+        ws_bytes = own_workspace(sr, dt, p, &optional);
+        if (ws_bytes > 0 && optional) {
+            // Under capture such a product runs without: no allocation nodes.
+            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+            if (hipStreamIsCapturing(st, &cap) != hipSuccess) (void)hipGetLastError();
+            if (cap != hipStreamCaptureStatusNone) ws_bytes = 0;
         }
         if (ws_bytes > 0) {
             TG_HIP(hipMallocAsync(&work, ws_bytes, st));
@@ -2055,6 +2082,21 @@ size_t tg_gemm_noalloc_bytes(tg_semiring semiring, tg_dtype dtype, tg_layout lay
     size_t ws_bytes = 0;
     const Plan pl = scratch_plan(semiring, dtype, p, &ws_bytes);
     return scratch_need(dtype, p, pl);
+}
+
+size_t tg_gemm_alloc_bytes(tg_semiring semiring, tg_dtype dtype, tg_layout layout, const void* A,
+                           const void* B, const void* C, const int32_t* argmax, int64_t batch,
+                           int64_t m, int64_t n, int64_t k, int64_t stride_a, int64_t stride_b,
+                           int64_t stride_c) {
+    const bool strided = stride_a != 0 || stride_b != 0 || stride_c != 0;
+    if (validate_forward(semiring, dtype, layout, A, B, C, batch, m, n, k, stride_a, stride_b,
+                         stride_c, strided) != TG_OK)
+        return ~size_t(0);
+    if (batch == 0 || m == 0 || n == 0) return 0;
+    const Problem p = make_problem(layout, A, B, const_cast<void*>(C), const_cast<int32_t*>(argmax),
+                                   batch, m, n, k, stride_a, stride_b, stride_c, strided);
+    bool optional;
+    return own_workspace(semiring, dtype, p, &optional);
 }
 
 size_t tg_gemm_workspace_size(tg_dtype dtype, int64_t batch, int64_t m, int64_t n, int64_t k,

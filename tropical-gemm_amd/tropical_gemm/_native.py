@@ -59,6 +59,8 @@ SIGNATURES = {
                        _i64, _i64, _vp, ctypes.POINTER(_i32)], _i32),
     "tg_gemm_small_plan": ([_i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
                             _i64, _i64], ctypes.c_char_p),
+    "tg_gemm_alloc_bytes": ([_i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
+                             _i64, _i64], _sz),
     "tg_gemm_workspace_size": ([_i32, _i64, _i64, _i64, _i64, _i32], _sz),
     "tg_gemm_ws": ([_i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _sz, _vp],
                    _i32),
