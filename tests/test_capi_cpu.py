@@ -254,3 +254,34 @@ def test_tg_gemm_allocates_a_workspace_where_it_pays(dt, batch, m, n, k, argmax,
                                   m * n)
     full = lib.tg_gemm_workspace_size(nat.DTYPE[dt], batch, m, n, k, int(argmax))
     assert got == (full if allocates else 0)
+
+
+@pytest.mark.parametrize("dt,batch,m,n,k,argmax,expected", [
+    # Sizes either side of where the direct-to-LDS tiles outweigh their
+    # prepasses and padding (expected: the start of the path's name).
+    ("f64", 1, 1000, 1000, 300, True, "tiles_exact"), ("f64", 1, 1000, 1000, 400, True, "dl64s"),
+    ("f64", 256, 64, 64, 512, True, "tiles_exact"), ("f64", 256, 64, 64, 513, True, "dl64s"),
+    ("f64", 1, 8, 65536, 512, True, "tiles_exact"), ("f64", 1, 1500, 1500, 256, True, "dl64s"),
+    ("f64", 64, 128, 128, 257, False, "tiles"), ("f64", 64, 128, 128, 320, False, "dl64s"),
+    ("f64", 1, 512, 512, 256, False, "dl64s"),
+    ("i64", 1, 1000, 1000, 300, True, "tiles_exact"), ("i64", 1, 1000, 1000, 513, True, "dl64s"),
+    ("i64", 128, 128, 128, 160, True, "tiles_exact"), ("i64", 128, 128, 128, 193, True, "dl64s"),
+    ("i64", 1024, 33, 33, 128, True, "tiles_exact"), ("i64", 1, 4096, 4096, 97, True, "dl64s"),
+    ("i64", 1, 1500, 1500, 100, False, "tiles"), ("i64", 1, 1500, 1500, 128, False, "dl64s"),
+    ("i64", 1, 1000, 1000, 65, False, "tiles"), ("i64", 1, 1000, 1001, 64, False, "dl64s"),
+    ("f32", 500, 65, 65, 97, True, "tiles_exact"), ("f32", 500, 65, 65, 200, True, "dl_elem"),
+    ("f32", 1, 1000, 1001, 97, True, "dl_elem"), ("i32", 100, 100, 101, 97, True, "tiles_exact"),
+    ("i32", 100, 100, 101, 130, True, "dl_elem"), ("f32", 1, 1000000, 2, 515, False, "tiles"),
+    ("i32", 500, 65, 65, 100, False, "tiles"), ("i32", 1, 700, 701, 100, False, "dl_elem"),
+    ("f32", 1, 3, 100000, 97, True, "dl_elem"),
+])
+def test_gemm_plan_either_side_of_the_64x64_tiles(dt, batch, m, n, k, argmax, expected):
+    strides = (m * k, k * n, m * n)
+    assert nat.gemm_plan("maxmul", dt, m, n, k, argmax, batch=batch,
+                         strides=strides).startswith(expected)
+
+
+def test_gemm_plan_of_unaligned_short_k_keys():
+    for m, n, k, expected in ((524288, 33, 12, "tiles_exact"), (524288, 33, 20, "kresg"),
+                              (65536, 33, 12, "kresg"), (524288, 48, 12, "kresg")):
+        assert nat.gemm_plan("maxplus", "i32", m, n, k, True) == expected

@@ -15,12 +15,16 @@ pytestmark = pytest.mark.gpu
 PLAN = {True: "dl64s_4x4_cl16", False: "dl64s_4x4"}
 
 # Up to 256 tiles K runs in three (argmax) or four slices, above in one or two.
-# (m, n, k): a last k-tile of 1, 2, 15 and 16 k, 17 and 18 k-tiles (slices of
+# (m, n, k): a last k-tile of 1, 2, 15 and 16 k, 33 and 34 k-tiles (slices of
 # unequal length), odd and even rows (element and 16-byte loads), ragged last
-# columns; 306 tiles; K below 256 (i64 only): 9 k-tiles leave the fourth slice
-# empty, 97 is the chunked mode's first K.
-SHAPES = [(513, 511, 257), (514, 516, 258), (449, 577, 271), (576, 514, 272), (512, 520, 288),
-          (1025, 1090, 257), (1030, 1026, 274), (513, 511, 130), (515, 512, 97)]
+# columns; 306 tiles; the first K of each rule; value-only i64 at 9 k-tiles (the
+# fourth slice empty).
+SHAPES = [(513, 511, 513), (514, 516, 514), (449, 577, 527), (576, 514, 528), (512, 520, 544),
+          (1025, 1090, 513), (1030, 1026, 530)]
+SHORT = {("f64", True): [(1473, 1500, 257), (1025, 1090, 385)],
+         ("f64", False): [(513, 519, 257), (449, 577, 320), (1025, 1090, 271)],
+         ("i64", True): [(1025, 1090, 193), (1473, 1501, 129), (2001, 2003, 97)],
+         ("i64", False): [(513, 511, 130), (515, 512, 81), (1025, 1090, 121)]}
 
 
 def _data(sr, dtype, m, n, k):
@@ -36,25 +40,45 @@ def _data(sr, dtype, m, n, k):
     return a.astype(dtype), b.astype(dtype)
 
 
-# f64 takes these tiles from K = 256.
-EDGES = [(dt, *s) for dt in ("f64", "i64") for s in SHAPES if dt == "i64" or s[2] >= 256]
-
-
-@pytest.mark.parametrize("dt,m,n,k", EDGES, ids=["-".join(map(str, e)) for e in EDGES])
-def test_dl64s_edges(dt, m, n, k):
+def _run(sr, dt, m, n, k, with_argmax, a, b, c_ref, am_ref):
+    """The product with a workspace of its full size (tg_gemm allocates one only
+    where it pays)."""
     from tropical_gemm import _native as nat
 
+    lib = nat.load()
+    assert nat.gemm_plan(sr, dt, m, n, k, with_argmax) == PLAN[with_argmax]
+    print(f"[case] dl64s {sr} {dt} {m}x{n}x{k} argmax={with_argmax}", flush=True)
+    ta, tb = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    c = torch.empty((m, n), dtype=ta.dtype, device="cuda")
+    am = torch.empty((m, n), dtype=torch.int32, device="cuda") if with_argmax else None
+    wsb = lib.tg_gemm_workspace_size(nat.DTYPE[dt], 1, m, n, k, int(with_argmax))
+    ws = torch.empty(max(wsb, 256), dtype=torch.uint8, device="cuda")
+    nat.check(lib.tg_gemm_ws(0, nat.SEMIRING[sr], nat.DTYPE[dt], 0, ta.data_ptr(), tb.data_ptr(),
+                             c.data_ptr(), None if am is None else am.data_ptr(), m, n, k,
+                             ws.data_ptr(), wsb, torch.cuda.current_stream().cuda_stream))
+    assert_exact(c.cpu().numpy(), None if am is None else am.cpu().numpy(), c_ref,
+                 am_ref if with_argmax else None)
+
+
+@pytest.mark.parametrize("dt", ["f64", "i64"])
+@pytest.mark.parametrize("m,n,k", SHAPES, ids=["x".join(map(str, s)) for s in SHAPES])
+def test_dl64s_edges(dt, m, n, k):
     for sr in tc.SEMIRINGS:
         a, b = _data(sr, tc.NP_DTYPES[dt], m, n, k)
         c_ref, am_ref = oracle.gemm(sr, a, b)
         for with_argmax in (True, False):
-            assert nat.gemm_plan(sr, dt, m, n, k, with_argmax) == PLAN[with_argmax]
-            print(f"[case] dl64s {sr} {dt} {m}x{n}x{k} argmax={with_argmax}", flush=True)
-            c, am = gpu_gemm(sr, a, b, with_argmax)
-            assert_exact(c, am, c_ref, am_ref if with_argmax else None)
+            _run(sr, dt, m, n, k, with_argmax, a, b, c_ref, am_ref)
 
 
-@pytest.mark.parametrize("m,n,k", [(513, 515, 259), (1090, 1024, 272)])
+@pytest.mark.parametrize("dt,with_argmax", list(SHORT), ids=[f"{d}-{w}" for d, w in SHORT])
+def test_dl64s_short_k(dt, with_argmax):
+    for q, (m, n, k) in enumerate(SHORT[dt, with_argmax]):
+        sr = tc.SEMIRINGS[q % 3]
+        a, b = _data(sr, tc.NP_DTYPES[dt], m, n, k)
+        _run(sr, dt, m, n, k, with_argmax, a, b, *oracle.gemm(sr, a, b))
+
+
+@pytest.mark.parametrize("m,n,k", [(513, 515, 515), (1090, 1024, 528)])
 @pytest.mark.parametrize("sr", tc.SEMIRINGS)
 def test_dl64s_nan_rule(sr, m, n, k):
     a, b = nan_inputs(sr, np.float64, m, n, k, seed=5)
@@ -73,7 +97,7 @@ def test_dl64s_wrapping_zeros_and_batches(dt):
     """Batch strides that break the 16-byte alignment; wrapping i64 sums,
     signed zeros and rows that never beat the tropical zero."""
     rng = np.random.default_rng(9)
-    m, n, k = 320, 330, 260
+    m, n, k = 320, 330, 520
     if dt == "i64":
         info = np.iinfo(np.int64)
         vals = np.array([0, 1, -1, info.max, info.min, info.max // 2 + 1], np.int64)

@@ -792,13 +792,22 @@ constexpr int64_t exact_tiles_max_k() {
 }
 
 // i64 argmax leaves the exact mode earlier where its chunked tiles run
-// tg_gemm_dl64s: from K = 97 on tiles at least half full, with the workspace
-// for B^T (us on MI355X, chunked / exact: 4096^2 x 128 429 / 548, 3001^2 x
-// 300 501 / 731, 2048^3 1159 / 2047; 2048^2 x 80 122 / 95).  Batches of small
-// products would mostly stage B^T.
+// tg_gemm_dl64s, with the workspace for B^T (us on MI355X, chunked / exact).  The
+// staging and the resolve weigh on short K, the more the fewer tiles there are:
+//   1024 tiles of 64 x 64 and more, of which few are partial, from K = 97: 4096^2
+//     x 128 429 / 548, 3001^2 x 300 501 / 731, 2048^3 1159 / 2047; narrower
+//     matrices 1024 x (33 x 33 x 128) 148 / 141, x 160 170 / 173;
+//   more than 512, 1500^2 x 100 98 / 86, x 128 104 / 105, x 188 128 / 150;
+//   more than 256, 128 x (128 x 128 x 160) 97 / 90, x 256 127 / 137;
+//   up to 256, whose exact mode is one round of the chip: 1000^2 x 188 63 / 53,
+//     x 300 82 / 81, x 512 114 / 133, 256 x (64 x 64 x 300) 95 / 81, x 512 133 / 134.
 template <typename T>
 bool chunked_i64(const Problem& p, size_t ws_bytes) {
-    if (!std::is_same<T, int64_t>::value || p.K <= 96 || p.M < 32 || p.N < 32) return false;
+    if (!std::is_same<T, int64_t>::value || p.M < 32 || p.N < 32) return false;
+    const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
+    const bool wide = p.M >= 512 && p.N >= 512;
+    const int64_t from = tiles64 <= 256 ? 513 : tiles64 <= 512 ? 193 : !wide ? 161 : tiles64 < 1024 ? 128 : 97;
+    if (p.K < from) return false;
     return ws_layout(TG_I64, p.batch, p.M, p.N, p.K, true, 1).total <= ws_bytes &&
            tg::dl64s_fits(p.M, p.N, p.K);
 }
@@ -868,14 +877,41 @@ int64_t dl64_tiles(const Problem& p) {
 //     240 43 / 85; wide 4096 x 1024 x 240 72 / 90, but 20000 x 200 x 240 133 /
 //     105, whose wave tiles fill 1.2 rounds of the chip's 4096 waves: from
 //     three quarters of the last round up.
+//   Column groups that are not 16-byte aligned, from 4 M outputs up (which then
+//     bound it), K >= 20: 524288 x 33 x 12 96 / 78, x 17 95 / 92, x 24 96 / 114.
 bool takes_kresg(const Problem& p) {
     if (!tg::kresg_fits(p.M, p.N, p.K) || p.M < 32) return false;
     const int64_t tiles = tg::kresg_wave_tiles(p.M, p.N) * p.batch;
     if (tiles < 64) return false;
+    if (p.N % 4 != 0 && p.K < 20 && double(p.batch) * double(p.M) * double(p.N) >= double(1 << 22))
+        return false;
     if (p.K <= 32) return (p.N <= 64 && p.K >= 12) || (p.N <= 256 && p.K >= 20);
     if (p.K <= 160) return true;
     const int64_t rounds = (tiles + 4095) / 4096;
     return 4 * tiles >= 3 * 4096 * rounds;
+}
+
+// True when too much of a 32-bit product's 64 x 64 x 32 element-load tiles is
+// padding for them, on more tiles than CUs (fewer make one round either way).
+// us on MI355X, element loads / generic kernel, whose tiles are 128 x 64:
+//   argmax: f32 500 x (65 x 65 x 97) 126 / 93, x 130 137 / 121, x 200 160 / 176,
+//     1000000 x 2 x 130 784 / 713; i32, whose exact mode is the faster one, 100 x
+//     (100 x 101 x 97) 43 / 38, x 130 47 / 48;
+//   value-only: i32 500 x (65 x 65 x 65) 45 / 36, x 130 69 / 64, x 200 94 / 93,
+//     50000 x 50 x 65 26 / 24, x 130 38 / 40; f32 300000 x 5 x 65 72 / 62, x 200
+//     146 / 155, 100000 x 33 x 65 29 / 32; four columns or fewer at any K: 1000000
+//     x 2 x 515 1256 / 1121.
+// A few rows are padding in the generic kernel too (3 x 100000 x 97 94 / 129).
+bool elem_padded(const Problem& p, int64_t tiles64, bool i32) {
+    if (p.M <= 16) return false;
+    const bool argmax = p.IDX != nullptr;
+    if (argmax && i32 && p.K < 128) return true;
+    if (!argmax && p.N <= 4) return true;
+    const double fill = double(p.batch) * double(p.M) * double(p.N) * double(p.K) /
+                        (double(tiles64) * 4096 * double((p.K + 31) / 32 * 32));
+    if (argmax) return fill < 0.22 && p.K < 160;
+    if (p.K < 64) return i32 && fill < 0.3 && p.K < 56;
+    return (p.K < 96 && fill < (i32 ? 0.7 : 0.3)) || (p.K < 200 && fill < 0.22);
 }
 
 // Chooses the kernel.  ws_bytes limits split K (the partials live in the
@@ -928,11 +964,13 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
         // 750, i32 455 / 807, 701^3 54 / 301, 3001 x 1501 x 301 102 / 182,
         // 3001^2 x 100 104 / 121, x 65 91 / 86 (so up to K = 96 the exact mode
         // stays); value-only 2001^3 291 / 342, 2001^2 x 60 15.5 / 22.8.  Below
-        // K = 48 most of a second k-tile would be padding.
+        // K = 48 most of a second k-tile would be padding.  More than a round of
+        // tiles whose work is mostly padding (elem_padded).
         const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
         const int slices = tg::dl_elem_slices(tiles64, p.K, argmax);
         auto take_elem = [&]() {
             if (tiles64 < 64 || !tg::dl_elem_fits<8>(p.M, p.N, p.K)) return false;
+            if (tiles64 > 256 && elem_padded(p, tiles64, std::is_same<T, int32_t>::value)) return false;
             if (!argmax) {
                 if (p.K < 48) return false;
                 pl.path = Path::DL_ELEM;
@@ -1039,7 +1077,11 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
         // argmax 1536^2 x 768 245 / 357, 1024^3 149 / 277, 2047 x 2049 x 1025
         // 518 / 1053, 3001^2 x 300 376 / 459, 3000 x 2000 x 256 221 / 250;
         // value-only 1536^2 x 768 200 / 263, 1024^3 111 / 203, 3001^2 x 300
-        // 249 / 323.
+        // 249 / 323.  Short K on few or narrow tiles stays on the generic kernel:
+        // argmax (exact mode) 1000^2 x 300 70 / 63, x 384 77 / 78, 1500^2 x 256
+        // 126 / 131, 256 x (64 x 64 x 512) 115 / 103, 8 x 65536 x 512 337 / 331;
+        // value-only 64 x (128 x 128 x 257) 62 / 56, 300 x 5000 x 300 73 / 69, x
+        // 384 84 / 85, 512^2 x 256 35 / 42.
         const int64_t tiles = dl64_tiles(p);
         const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
         if (p.K >= 256 && dl64_ws_bytes(p.batch, p.M, p.N, p.K, argmax) <= ws_bytes) {
@@ -1048,18 +1090,27 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
                 pl.path = argmax ? Path::DL64 : Path::DL64_VALUE;
                 return pl;
             }
-            if (tiles64 >= 64 && tg::dl64s_fits(p.M, p.N, p.K)) {
+            const int64_t narrow = p.M < p.N ? p.M : p.N;
+            const bool enough = !argmax ? p.K >= 320 || narrow >= 512
+                                : p.K > exact_tiles_max_k<T>() ||
+                                      (narrow >= 128 && (tiles64 > 512 || p.K > 384));
+            if (enough && tiles64 >= 64 && tg::dl64s_fits(p.M, p.N, p.K)) {
                 pl.path = argmax ? Path::DL64S : Path::DL64S_VALUE;
                 return pl;
             }
         }
     }
     // i64: the chunked and the value-only tiles are tg_gemm_dl64s; the
-    // register-staged kernel keeps sizes it does not fit and value-only K below
-    // 64 (2048^2 x 80: 52 us both).
+    // register-staged kernel keeps sizes it does not fit and value-only short K
+    // (us, dl64s / tiles: one round of tiles 1000^2 x 64 15 / 17, x 65 18.7 / 17.8, x
+    // 80 18 / 21; more 1500^2 x 100 53 / 50, x 128 57 / 61, 128 x (128 x 128 x 64)
+    // 26 / 24).
     const bool i64_dl = std::is_same<T, int64_t>::value && tg::dl64s_fits(p.M, p.N, p.K);
+    const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
     if (!argmax)
-        pl.path = i64_dl && p.K >= 64 ? Path::DL64S_I64_VALUE : Path::TILES;
+        pl.path = i64_dl && (tiles64 <= 256 ? p.K >= 80 || p.K == 64 : p.K >= 120)
+                      ? Path::DL64S_I64_VALUE
+                      : Path::TILES;
     else if (exact || (p.K <= exact_tiles_max_k<T>() && !chunked_i64<T>(p, ws_bytes)))
         pl.path = Path::TILES_EXACT;
     else
@@ -1351,11 +1402,11 @@ bool workspace_optional(tg_semiring sr, tg_dtype dt, const Problem& p, const Pla
 // allocate and free it.  Between synchronisations the stream's pool keeps up to
 // 2 MB; beyond that a call that is waited for pays about 25 us and 2.5 us per MB
 // (MI355X), against what the path gains.  us, with the allocation / without a
-// workspace: f32 argmax 16 x (64 x 1025 x 97) 63 / 49, x 200 79 / 93, 50000 x 50
-// x 384 285 / 176, 1000 x 1001 x 97 (0.4 MB) 37 / 48; f64 argmax 1500^2 x 300 164
-// / 152, x 512 216 / 254, 128 x (128 x 128 x 512) 288 / 178; i64 argmax 1500^2 x
-// 188 159 / 150, x 300 209 / 235, 1000^3 223 / 256, 256 x (64 x 64 x 1000) 316 /
-// 257.
+// workspace: f32 argmax 16 x (64 x 1025 x 97) 78 / 60, x 200 89 / 105, 50000 x 50
+// x 384 303 / 187, 1000 x 1001 x 97 (0.4 MB) 46 / 59; f64 argmax 1500^2 x 300 176
+// / 163, x 512 225 / 264, 128 x (128 x 128 x 512) 306 / 190; i64 argmax 1500^2 x
+// 188 170 / 161, x 300 216 / 245, 1000^3 231 / 267, 256 x (64 x 64 x 1000) 330 /
+// 268.
 bool allocation_pays(tg_dtype dt, const Problem& p, size_t bytes) {
     constexpr size_t kMB = size_t(1) << 20;
     if (bytes <= 2 * kMB || p.IDX == nullptr) return true;
