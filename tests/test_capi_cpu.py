@@ -237,7 +237,9 @@ def test_noalloc_scratch_where_no_kernel_is_without():
 
 @pytest.mark.parametrize("dt,batch,m,n,k,argmax,allocates", [
     # Tiles without a workspace, where one would have to be allocated per call.
-    ("f32", 16, 64, 1025, 97, True, False), ("f32", 16, 64, 1025, 200, True, True),
+    ("f32", 16, 64, 1025, 97, True, False), ("f32", 16, 64, 1025, 300, True, True),
+    ("f32", 500, 65, 65, 200, True, False), ("i32", 30, 129, 131, 255, True, False),
+    ("i32", 64, 33, 65, 97, True, False), ("f64", 1, 1000, 1000, 257, False, False),
     ("f32", 1, 50000, 50, 384, True, False), ("f32", 1, 1000, 1001, 97, True, True),
     ("f64", 1, 1500, 1500, 300, True, False), ("f64", 1, 1500, 1500, 512, True, True),
     ("f64", 128, 128, 128, 512, True, False), ("f64", 1, 1000, 1000, 512, False, True),

@@ -1399,22 +1399,25 @@ bool workspace_optional(tg_semiring sr, tg_dtype dt, const Problem& p, const Pla
 }
 
 // Whether an optional workspace of this size pays when the call itself has to
-// allocate and free it.  Between synchronisations the stream's pool keeps up to
-// 2 MB; beyond that a call that is waited for pays about 25 us and 2.5 us per MB
-// (MI355X), against what the path gains.  us, with the allocation / without a
-// workspace: f32 argmax 16 x (64 x 1025 x 97) 78 / 60, x 200 89 / 105, 50000 x 50
-// x 384 303 / 187, 1000 x 1001 x 97 (0.4 MB) 46 / 59; f64 argmax 1500^2 x 300 176
-// / 163, x 512 225 / 264, 128 x (128 x 128 x 512) 306 / 190; i64 argmax 1500^2 x
-// 188 170 / 161, x 300 216 / 245, 1000^3 231 / 267, 256 x (64 x 64 x 1000) 330 /
-// 268.
+// allocate and free it: about 8 us for a call that is waited for while the
+// stream's pool keeps it between synchronisations (up to 2 MB), beyond that
+// 25 us and 2.5 us per MB (MI355X), against what the path gains.  us, with the
+// allocation / without a workspace: f32 argmax 1000 x 1001 x 97 (0.4 MB) 46 / 59,
+// 16 x (64 x 1025 x 97) 78 / 60, 500 x (65 x 65 x 200) 206 / 189, 50000 x 50 x 384
+// 303 / 187; i32, whose exact mode is the faster one, 64 x (33 x 65 x 97) 52 / 44,
+// 30 x (129 x 131 x 255) 106 / 97; f64 argmax 1500^2 x 300 176 / 163, x 512 225 /
+// 264, 128 x (128 x 128 x 512) 306 / 190, value-only 1000^2 x 257 63 / 55, 300 x
+// 5000 x 384 104 / 97; i64 argmax 1500^2 x 188 170 / 161, x 300 216 / 245, 1000^3
+// 231 / 267, 256 x (64 x 64 x 1000) 330 / 268.
 bool allocation_pays(tg_dtype dt, const Problem& p, size_t bytes) {
     constexpr size_t kMB = size_t(1) << 20;
-    if (bytes <= 2 * kMB || p.IDX == nullptr) return true;
     const int64_t narrow = p.M < p.N ? p.M : p.N;
+    if (p.IDX == nullptr) return p.K >= (narrow >= 512 ? 300 : 400);
+    if (bytes <= 2 * kMB) return dt != TG_I32 || p.K >= 128;
     const double products = double(p.batch) * double(p.M) * double(p.N) * double(p.K);
     if (dt == TG_F64) return narrow >= 256 && products >= 8e8;
     if (dt == TG_I64) return narrow >= 256 && (p.K >= 800 || products >= 5.5e8);
-    return p.K >= 192 ? bytes <= 64 * kMB || narrow >= 128 : narrow >= 512;
+    return p.K >= (dt == TG_I32 ? 320 : 256) ? bytes <= 64 * kMB || narrow >= 128 : narrow >= 512;
 }
 
 // Bytes that tg_gemm allocates for the call: the full workspace, for the
