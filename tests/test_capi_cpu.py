@@ -287,3 +287,31 @@ def test_gemm_plan_of_unaligned_short_k_keys():
     for m, n, k, expected in ((524288, 33, 12, "tiles_exact"), (524288, 33, 20, "kresg"),
                               (65536, 33, 12, "kresg"), (524288, 48, 12, "kresg")):
         assert nat.gemm_plan("maxplus", "i32", m, n, k, True) == expected
+
+
+@pytest.mark.parametrize("sr,dt,batch,m,n,k,argmax,few", [
+    # Long K of few outputs: 32-bit K that splits over the whole chip goes there.
+    ("maxplus", "f32", 1, 256, 256, 4096, False, True), ("maxplus", "f32", 1, 256, 256, 8192, False, False),
+    ("maxplus", "f32", 1, 256, 256, 4096, True, True), ("maxplus", "i32", 1, 256, 256, 8192, True, False),
+    ("maxplus", "f32", 1, 700, 700, 1024, False, False), ("maxplus", "f32", 1, 700, 700, 1024, True, True),
+    ("maxplus", "f32", 1, 64, 64, 1 << 20, False, False), ("maxplus", "f32", 1, 64, 64, 32768, False, True),
+    ("maxplus", "i32", 1, 64, 64, 65536, False, False), ("maxplus", "f32", 1, 64, 64, 65536, True, True),
+    ("maxplus", "f32", 1, 16, 256, 32768, False, True), ("maxplus", "f32", 1, 16, 256, 65536, False, False),
+    ("maxplus", "f32", 1, 16, 16, 65536, True, True), ("maxplus", "f32", 1, 16, 16, 262144, True, False),
+    ("maxplus", "f32", 1, 64, 64, (1 << 20) - 1, False, True),  # K that does not split
+    ("maxplus", "f64", 1, 64, 64, 1 << 20, True, True),
+    ("maxplus", "f32", 256, 48, 48, 512, True, False), ("maxplus", "f32", 64, 48, 48, 512, True, True),
+    # Up to 64 columns at short K.
+    ("maxplus", "f32", 1, 524288, 64, 2, True, False), ("maxplus", "f32", 1, 524288, 64, 12, True, True),
+    ("maxplus", "f32", 1, 524288, 32, 2, True, True), ("maxplus", "f32", 1, 524288, 33, 32, True, False),
+    ("maxplus", "f32", 1, 524288, 3, 2, True, False), ("maxplus", "f32", 1, 524288, 3, 12, True, True),
+    ("maxplus", "f64", 1, 524288, 33, 24, True, False), ("maxplus", "f64", 1, 65536, 30, 12, True, True),
+    ("maxplus", "f32", 1, 524288, 33, 32, False, False), ("maxplus", "f64", 1, 524288, 50, 12, False, True),
+    ("maxplus", "f32", 5000, 48, 48, 8, False, False), ("maxplus", "f32", 5000, 48, 48, 16, False, True),
+    ("maxplus", "f32", 1, 4096, 33, 32, True, True),
+    ("maxplus", "f32", 1, 3, 524288, 36, False, False), ("maxplus", "f32", 1, 524288, 8, 36, False, True),
+])
+def test_few_output_kernel_leaves_what_others_run_faster(sr, dt, batch, m, n, k, argmax, few):
+    plan = nat.gemm_small_plan(sr, dt, m, n, k, argmax, batch=batch,
+                               strides=(m * k, k * n, m * n))
+    assert ("waves" in plan) == few, plan

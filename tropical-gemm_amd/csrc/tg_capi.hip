@@ -1490,6 +1490,56 @@ tg::SmallProblem small_problem(tg_semiring sr, tg_dtype dt, const Problem& p) {
                             p.sA, p.sB, p.sC};
 }
 
+int64_t tiles64_of(const Problem& p) { return ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch; }
+
+// True when the few-output kernel is the faster one for any number of outputs
+// up to 64 columns wide at K <= 32.  The others write 256-column (short K, for
+// aligned columns) or 64-column tiles, mostly padding there, but short K makes
+// the outputs themselves the bound, which they write in longer runs.  us on
+// MI355X, small / other:
+//   aligned, argmax: f32 524288 x 64 x 2 114 / 60, x 8 160 / 128, x 12 170 / 190;
+//     N <= 32 from K = 2; value-only from K = 3 beyond 32 columns (f64 524288 x 64
+//     x 1 65 / 53), batches of few rows from 12 (f32 5000 x (48 x 48 x 8) 54 / 44, x
+//     16 31 / 66);
+//   any columns, argmax: beyond 32 never (524288 x 33 f32 x 32 182 / 125, f64 x 24
+//     299 / 162); up to 16 f32 524288 x 3 x 2 48 / 30, x 12 47 / 54, f64 x 9 x 8
+//     61 / 84; between, f32 x 21 x 24 99 / 96, x 32 107 / 115, f64 65536 x 30 x 12
+//     15 / 18, x 17 x 17 22 / 20; value-only beyond 32 up to K = 16 (524288 x 50 f64
+//     x 12 86 / 143, x 32 250 / 209).
+bool small_takes_narrow(tg_dtype dt, const Plan& pl, const Problem& p) {
+    const bool aligned = pl.path == Path::SHORTK, wide = dt == TG_F64 || dt == TG_I64;
+    if (p.IDX == nullptr) {
+        if (p.N <= 32) return true;
+        return aligned ? p.K >= (p.batch > 1 && p.M < 64 ? 12 : 3) : p.K <= 16;
+    }
+    if (aligned) return p.K >= (p.N <= 32 ? 2 : 12);
+    if (p.N <= 16) return p.K >= (wide ? 5 : 10);
+    if (p.N <= 32) return wide ? p.K <= 16 : dt == TG_F32 && p.K >= 28;
+    return false;
+}
+
+// True when a 32-bit product whose K the direct-to-LDS kernel splits over the
+// whole chip (into launches, with a merge) is past the few-output kernel's K: a
+// tile's waves there are at most 16.  us on MI355X, small / split, by K times
+// the outputs of the split kernel's tiles: value-only f32 256^2 x 4096 (2.7e8)
+// 19 / 29, x 8192 37 / 34, 512^2 x 1024 19 / 25, x 2048 (5.4e8) 33 / 27, 700^2 x 1024
+// (5.1e8) 36 / 26, 128^2 x 32768 (5.4e8) 53 / 65, x 65536 99 / 82; argmax 256^2 x
+// 8192 (5.4e8) 51 / 57, x 16384 96 / 82, i32 29 / 43 at 4096 (2.7e8), 75 / 66 at
+// 8192.  One tile, value-only: 64^2 x 32768 52 / 67, x 65536 101 / 101, i32 98 /
+// 84.  Up to 16 rows or columns that is mostly padding: 16 x 256 x 32768
+// value-only 59 / 69, x 65536 115 / 88, 16^2 x 65536 argmax 72 / 113, x 262144 263 /
+// 239.
+bool split_outruns_small(const Plan& pl, const Problem& p) {
+    const bool argmax = p.IDX != nullptr;
+    const bool slices_ok = pl.path == Path::DL_44_8 || pl.path == Path::DL_44_16;
+    if (pl.splits <= 1 || wg_slices(slices_ok, argmax, pl.splits, p.K) > 0) return false;
+    const int64_t tiles64 = tiles64_of(p);
+    if (tiles64 * pl.splits < 256) return false;
+    if (p.M <= 16 || p.N <= 16) return p.K > (argmax ? 65536 : 32768);
+    return (!argmax && p.K > 49152) ||
+           double(p.K) * double(tiles64 * 4096) > (argmax ? 4.5e8 : 3.5e8);
+}
+
 // Outputs (batch x M x N) below which the few-output kernel (tg_gemm_small.hpp)
 // is the faster one, by the path the problem would take otherwise.  Measured
 // on MI355X over 290 shapes of every dtype, with and without argmax (small /
@@ -1516,6 +1566,8 @@ tg::SmallProblem small_problem(tg_semiring sr, tg_dtype dt, const Problem& p) {
 //   i64: argmax 1536^2 x 768 340 / 365, 2047 x 2049 x 1025 780 / 803, 2048^3
 //     1490 / 1160, in the exact mode's range 2048^2 x 80 83 / 95; value-only
 //     2047 x 2049 x 1025 586 / 652, 3001^2 x 300 388 / 349.
+//   K slices in one workgroup on most of the CUs: 256 x (48 x 48 x 512) argmax f32
+//     53 / 46, i32 62 / 52, 64 x (48 x 48 x 512) 21 / 37, 700^2 x 1024 45 / 52.
 int64_t small_output_limit(tg_dtype dt, const Plan& pl, const Problem& p) {
     constexpr int64_t k1 = int64_t(1) << 10;
     const bool argmax = p.IDX != nullptr;
@@ -1523,9 +1575,13 @@ int64_t small_output_limit(tg_dtype dt, const Plan& pl, const Problem& p) {
     if (pl.path == Path::KRESG)
         return p.K <= 32 ? 192 * k1 : p.K <= 48 ? 384 * k1 : p.K <= 160 ? 768 * k1 : 1280 * k1;
     if (p.K <= 32) {
-        if (p.N <= 64) return INT64_MAX;
+        if (p.N <= 64 && small_takes_narrow(dt, pl, p)) return INT64_MAX;
         return !argmax ? 512 * k1 : dt == TG_F64 ? 128 * k1 : 256 * k1;
     }
+    // Few rows of the short-K kernel's wide tiles, which it writes in 1 KB runs
+    // (3 x 524288 x 33 value-only 43 / 28, 16 rows 40 / 30).
+    if (pl.path == Path::SHORTK && p.N > 16) return 512 * k1;
+    if (split_outruns_small(pl, p)) return 0;
     if (narrow <= 16) return INT64_MAX;  // tiles of the other kernels are mostly padding
     switch (pl.path) {
         case Path::SHORTK: return 512 * k1;
@@ -1548,7 +1604,8 @@ int64_t small_output_limit(tg_dtype dt, const Plan& pl, const Problem& p) {
             if (pl.slices == 1) return 1280 * k1;
             return argmax ? 640 * k1 : dt == TG_F32 ? 512 * k1 : 768 * k1;
         default:  // direct-to-LDS, 32-bit
-            return narrow <= 32 ? 2048 * k1 : p.K >= 256 ? 640 * k1 : 512 * k1;
+            if (narrow <= 32) return 2048 * k1;
+            return p.K < 256 ? 512 * k1 : pl.splits > 1 && tiles64_of(p) > 160 ? 448 * k1 : 640 * k1;
     }
     if (dt == TG_I64)
         return pl.path == Path::TILES_EXACT ? 8192 * k1 : 4096 * k1;
