@@ -90,16 +90,33 @@ def _check(sr, items, with_argmax, **kw):
 
 # (batch, m, n, k), form: tiles of 4 x 16 (one row, ragged columns, K below,
 # at and past a step of 64 or 32 k), 8 x 16, 16 x 16 and 32 x 32 outputs, the
-# one-column form (N < 4), and K split over up to 16 waves.
+# one-column form (N < 4), and K split over up to 16 waves.  Every form runs with
+# and without argmax in every dtype (test_every_form_has_its_shapes).
 SHAPES = [
     ((1, 1, 5, 1), "4x16 waves 1"), ((1, 3, 16, 63), "4x16"), ((1, 5, 17, 65), "4x16"),
     ((1, 67, 45, 131), "4x16"), ((1, 4, 1000, 4096), "4x16"), ((1, 16, 777, 1500), "4x16"),
     ((3, 100, 260, 33), "8x16"), ((1, 130, 515, 97), "8x16"),
     ((1, 250, 900, 129), "16x16"), ((20, 63, 49, 700), "8x16"),
     ((30, 129, 131, 30), "32x32"), ((9, 300, 200, 127), "32x32"),
+    ((1, 20001, 31, 15), "32x32"), ((1, 20001, 31, 29), "32x32"),
     ((1, 1, 1, 7), "16x4"), ((1, 2, 3, 64), "16x4"), ((1, 1000, 1, 515), "16x4"),
     ((4, 33, 2, 2050), "16x4"),
 ]
+
+
+# The shapes that other kernels run faster: (dtype, with_argmax) by shape.
+OTHERS = {
+    (30, 129, 131, 30): {("f32", True), ("f64", True), ("i32", True), ("i64", True)},
+    (9, 300, 200, 127): {("f64", True)},
+    (1, 20001, 31, 15): {("f32", True), ("i32", True)},
+    (1, 20001, 31, 29): {("f64", True), ("i32", True), ("i64", True)},
+}
+
+
+def test_every_form_has_its_shapes():
+    ran = {(form.split()[0], dt, am) for shape, form in SHAPES for dt in ("f32", "f64", "i32", "i64")
+           for am in (True, False) if (dt, am) not in OTHERS.get(shape, ())}
+    assert len(ran) == 5 * 4 * 2
 
 
 @pytest.mark.parametrize("dt", ["f32", "f64", "i32", "i64"])
@@ -118,7 +135,8 @@ def test_small_forms(dt, shape, form):
         for with_argmax in (True, False):
             plan = nat.gemm_small_plan(sr, dt, m, n, k, with_argmax, batch=batch,
                                        strides=(m * k + 1, k * n + 1, m * n + 1), addresses=(8,) * 4)
-            if plan == "none":  # outside the kernel's range for this type
+            if (dt, with_argmax) in OTHERS.get(shape, ()):
+                assert plan == "none"
                 continue
             assert plan.startswith(form), plan
             print(f"[case] small {sr} {dt} {shape} argmax={with_argmax} {plan}", flush=True)

@@ -22,7 +22,7 @@ def _lib():
 
 def _operands(sr, dt, m, n, k, seed):
     rng = np.random.default_rng(seed)
-    dtype = {"f32": np.float32, "f64": np.float64, "i32": np.int32}[dt]
+    dtype = tc.NP_DTYPES[dt]
     if sr == "maxmul":
         return ((1.0 - rng.random((m, k))).astype(dtype),
                 (1.0 - rng.random((k, n))).astype(dtype))
@@ -66,6 +66,16 @@ CASES = [
     ("minplus", "f64", "row", False, (1024, 4096, 640), (1024, 2048, 576), "dl64_4x8"),
     ("maxplus", "i32", "col", True, (384, 256, 1024), (256, 128, 512), None),
     ("maxplus", "f32", "row", True, (3072, 4096, 1024), (512, 256, 512), "dl_4x8_cl16"),
+    # 64 x 64 tiles with element loads and of the 64-bit types, on the scratch
+    # (from the K no kernel without a workspace takes) and without it.
+    ("maxplus", "f32", "row", True, (1000, 1001, 400), (513, 511, 390), "dl_elem_cl8 slices 2"),
+    ("minplus", "f32", "row", True, (700, 701, 300), (513, 511, 290), "dl_elem_cl8 slices 2"),
+    ("maxplus", "f32", "row", False, (700, 701, 300), (513, 511, 97), "dl_elem slices 4"),
+    ("minplus", "f64", "row", True, (640, 641, 520), (513, 514, 515), "dl64s_4x4_cl16"),
+    ("maxplus", "f64", "row", False, (700, 701, 400), (513, 513, 321), "dl64s_4x4"),
+    ("maxplus", "i64", "row", True, (513, 514, 2050), (400, 300, 2049), "dl64s_4x4_cl16"),
+    ("maxplus", "i64", "col", True, (513, 514, 600), (400, 300, 520), "dl64s_4x4_cl16"),
+    ("maxplus", "i32", "row", True, (2000, 130, 61), (335, 254, 50), "kresg"),
 ]
 
 
@@ -79,7 +89,7 @@ def test_noalloc_matches_tg_gemm_twice(sr, dt, layout, argmax, first, second, pa
         pytest.skip("no GPU")
     lib = _lib()
     dev = torch.device("cuda", 0)
-    tdt = {"f32": torch.float32, "f64": torch.float64, "i32": torch.int32}[dt]
+    tdt = {"f32": torch.float32, "f64": torch.float64, "i32": torch.int32, "i64": torch.int64}[dt]
     stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     p = lambda t: None if t is None else ctypes.c_void_p(t.data_ptr())  # noqa: E731
     if path is not None:
