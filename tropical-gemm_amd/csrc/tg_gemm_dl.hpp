@@ -371,8 +371,9 @@ __global__ __launch_bounds__(TG_THREADS * HALVES) __attribute__((amdgpu_waves_pe
     // Split K: slice y covers k in [y*KS, (y+1)*KS) and writes its (value,
     // argmax) partial at C/IDX + y*sY (tg_merge_splits combines them).  An
     // unsplit launch has gridDim.y == 1, KS == K and sY == 0.  With
-    // halves, half h is slice h (KS == K / HALVES) and the halves merge in
-    // LDS into C/IDX (sY unused).
+    // halves, half h is slice h and the halves merge in LDS into C/IDX (sY
+    // unused): KS == K / HALVES for 16-byte loads, for element loads the
+    // k-tiles / HALVES rounded up, in k (the last slices shorter or empty).
     const int64_t y = HALVES > 1 ? half : int64_t(blockIdx.y);
     C += z * sC + (HALVES > 1 ? 0 : y * sY);
     if (ARGMAX) {

@@ -15,8 +15,10 @@
 //   alignment  16-byte loads and stores at 4-byte alignment.
 // Row tiles or panels outside the f32-key range (|x| >= 2^15) take the exact
 // per-product rule over the same tiles.
-// Bound: on ordinary K the LDS reads of the fragments (8 floats per 16 products
-// of a lane) beside the add + max3 chain, at short K the writes of C and argmax.
+// Bound: on ordinary K VALU issue, on the products of whole tiles (K to a
+// multiple of 32, N of 64: 1.64 times those of 100 states, 1.13 instructions per
+// ideal one of them), beside the LDS reads of the fragments (8 floats per 16
+// products of a lane); at short K the writes of C and argmax.
 // Measured on MI355X (us; before it: the generic kernel's exact mode,
 // direct-to-LDS or short-K tiles): 262144 x 16 x 16 27 (130), x 32 x 32 27
 // (234), x 48 x 48 45 (99), x 100 x 100 155 (364),
