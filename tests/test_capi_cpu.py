@@ -251,7 +251,8 @@ def test_noalloc_scratch_where_no_kernel_is_without():
 ])
 def test_tg_gemm_allocates_a_workspace_where_it_pays(dt, batch, m, n, k, argmax, allocates):
     lib = nat.load()
-    got = lib.tg_gemm_alloc_bytes(nat.SEMIRING["maxmul"], nat.DTYPE[dt], nat.LAYOUT["row"], 256,
+    sr = "maxplus" if dt == "i64" else "maxmul"
+    got = lib.tg_gemm_alloc_bytes(nat.SEMIRING[sr], nat.DTYPE[dt], nat.LAYOUT["row"], 256,
                                   256, 256, 256 if argmax else None, batch, m, n, k, m * k, k * n,
                                   m * n)
     full = lib.tg_gemm_workspace_size(nat.DTYPE[dt], batch, m, n, k, int(argmax))
@@ -265,22 +266,48 @@ def test_tg_gemm_allocates_a_workspace_where_it_pays(dt, batch, m, n, k, argmax,
     ("f64", 256, 64, 64, 512, True, "tiles_exact"), ("f64", 256, 64, 64, 513, True, "dl64s"),
     ("f64", 1, 8, 65536, 512, True, "tiles_exact"), ("f64", 1, 1500, 1500, 256, True, "dl64s"),
     ("f64", 64, 128, 128, 257, False, "tiles"), ("f64", 64, 128, 128, 320, False, "dl64s"),
+    ("f64", 128, 128, 128, 449, True, "tiles_exact"), ("f64", 128, 128, 128, 449, False, "tiles"),
+    ("f64", 128, 128, 128, 450, False, "dl64s"), ("f64", 1, 34, 47910, 321, False, "dl64s"),
+    ("f64", 1, 1501, 1501, 256, True, "tiles_exact"), ("f64", 1, 1501, 1501, 257, True, "dl64s"),
     ("f64", 1, 512, 512, 256, False, "dl64s"),
     ("i64", 1, 1000, 1000, 300, True, "tiles_exact"), ("i64", 1, 1000, 1000, 513, True, "dl64s"),
-    ("i64", 128, 128, 128, 160, True, "tiles_exact"), ("i64", 128, 128, 128, 193, True, "dl64s"),
+    ("i64", 128, 128, 128, 256, True, "tiles_exact"), ("i64", 128, 128, 128, 257, True, "dl64s"),
+    ("i64", 1, 34, 47910, 193, True, "tiles_exact"), ("i64", 1220, 64, 64, 257, True, "dl64s"),
     ("i64", 1024, 33, 33, 128, True, "tiles_exact"), ("i64", 1, 4096, 4096, 97, True, "dl64s"),
     ("i64", 1, 1500, 1500, 100, False, "tiles"), ("i64", 1, 1500, 1500, 128, False, "dl64s"),
-    ("i64", 1, 1000, 1000, 65, False, "tiles"), ("i64", 1, 1000, 1001, 64, False, "dl64s"),
+    ("i64", 1, 1500, 1500, 129, False, "tiles"), ("i64", 1, 1500, 1500, 192, False, "dl64s"),
+    ("i64", 1, 1000, 1000, 81, False, "tiles"), ("i64", 1, 1000, 1001, 64, False, "dl64s"),
     ("f32", 500, 65, 65, 97, True, "tiles_exact"), ("f32", 500, 65, 65, 200, True, "dl_elem"),
     ("f32", 1, 1000, 1001, 97, True, "dl_elem"), ("i32", 100, 100, 101, 97, True, "tiles_exact"),
     ("i32", 100, 100, 101, 130, True, "dl_elem"), ("f32", 1, 1000000, 2, 515, False, "tiles"),
-    ("i32", 500, 65, 65, 100, False, "tiles"), ("i32", 1, 700, 701, 100, False, "dl_elem"),
+    ("i32", 500, 65, 65, 100, False, "tiles"), ("i32", 1, 2001, 2001, 97, False, "tiles"),
+    ("i32", 1260, 85, 31, 131, False, "tiles"), ("f32", 53, 214, 388, 115, True, "tiles_exact"), ("i32", 1, 700, 701, 100, False, "dl_elem"),
     ("f32", 1, 3, 100000, 97, True, "dl_elem"),
 ])
 def test_gemm_plan_either_side_of_the_64x64_tiles(dt, batch, m, n, k, argmax, expected):
+    # i32 by MaxMul (MaxPlus argmax runs on keys there), i64 by MaxPlus (MaxMul has
+    # lines of its own).
+    sr = "maxplus" if dt == "i64" else "maxmul"
     strides = (m * k, k * n, m * n)
-    assert nat.gemm_plan("maxmul", dt, m, n, k, argmax, batch=batch,
-                         strides=strides).startswith(expected)
+    assert nat.gemm_plan(sr, dt, m, n, k, argmax, batch=batch, strides=strides).startswith(expected)
+
+
+@pytest.mark.parametrize("batch,m,n,k,expected", [
+    (1, 1500, 1500, 300, "tiles_exact"), (1, 1500, 1500, 301, "dl64s"),
+    (1, 34, 47910, 1500, "tiles_exact"), (1, 34, 47910, 1502, "dl64s"),
+    (1, 34, 47910, 1501, "tiles_exact"), (1, 100, 16383, 2500, "tiles_chunked"),
+    (1, 1378, 1379, 400, "tiles_exact"), (1, 1378, 1379, 513, "dl64s"),
+    (1, 1000, 1001, 512, "tiles_exact"), (1, 1000, 1001, 513, "dl64s"),
+])
+def test_gemm_plan_of_i64_maxmul_argmax(batch, m, n, k, expected):
+    assert nat.gemm_plan("maxmul", "i64", m, n, k, True, batch=batch).startswith(expected)
+
+
+def test_aligned_products_of_two_rounds_of_tiles():
+    for dt, k, argmax, expected in (("f32", 256, True, "dl_elem"), ("i32", 256, True, "dl_4x4"),
+                                    ("i32", 320, True, "dl_elem"), ("f32", 288, False, "dl_4x4"),
+                                    ("f32", 320, False, "dl_elem")):
+        assert nat.gemm_plan("maxplus", dt, 1408, 1408, k, argmax).startswith(expected)
 
 
 def test_gemm_plan_of_unaligned_short_k_keys():

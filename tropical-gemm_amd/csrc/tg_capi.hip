@@ -791,22 +791,39 @@ constexpr int64_t exact_tiles_max_k() {
     return sizeof(T) == 4 ? 384 : std::is_same<T, int64_t>::value ? 2048 : 512;
 }
 
+// More than a round of tg_gemm_dl64s tiles by element loads on matrices narrower
+// than 512.
+bool narrow_elements(const Problem& p) {
+    return (p.M < 512 || p.N < 512) && ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch > 256 &&
+           !tg::dl64s_vectors(p.N, p.K, p.sA, p.sB, p.A, p.B);
+}
+
 // i64 argmax leaves the exact mode earlier where its chunked tiles run
 // tg_gemm_dl64s, with the workspace for B^T (us on MI355X, chunked / exact).  The
-// staging and the resolve weigh on short K, the more the fewer tiles there are:
-//   1024 tiles of 64 x 64 and more, of which few are partial, from K = 97: 4096^2
-//     x 128 429 / 548, 3001^2 x 300 501 / 731, 2048^3 1159 / 2047; narrower
-//     matrices 1024 x (33 x 33 x 128) 148 / 141, x 160 170 / 173;
-//   more than 512, 1500^2 x 100 98 / 86, x 128 104 / 105, x 188 128 / 150;
-//   more than 256, 128 x (128 x 128 x 160) 97 / 90, x 256 127 / 137;
-//   up to 256, whose exact mode is one round of the chip: 1000^2 x 188 63 / 53,
-//     x 300 82 / 81, x 512 114 / 133, 256 x (64 x 64 x 300) 95 / 81, x 512 133 / 134.
-template <typename T>
+// staging and the resolve weigh on short K, the more the fewer and the narrower
+// the tiles are:
+//   up to 256 tiles of 64 x 64, whose exact mode is one round of the chip: 1000^2 x
+//     188 63 / 53, x 300 82 / 81, x 512 115 / 133, 256 x (64 x 64 x 512) 134 / 134;
+//   up to 512, or narrow, 128 x (128 x 128 x 193) 114 / 110, x 257 140 / 143, 64 x
+//     22528 x 193 115 / 107, x 257 138 / 139; 34 x 47910 x 161 145 / 137, x 225 183 / 185,
+//     1220 x (64 x 64 x 161) 263 / 226, x 300 0.90 times;
+//   beyond, wide: 1501^2 x 128 114 / 113, x 161 124 / 140; from 2048 tiles 3001^2 x 97
+//     251 / 272 (2001 x 2003 x 97 127 / 124).
+// MaxMul, whose 64-bit products the resolve computes once more (chunked / exact):
+// 1500^2 x 193 186 / 165, x 301 249 / 252, 3001^2 x 225 563 / 563; narrower 128 x (128
+// x 128 x 1025) 664 / 583, x 1500 834 / 869, 34 x 47910 x 1500 1296 / 1270 (by element loads 100 x
+// 16383 x 2500 1485 / 1368 on the register-staged tiles); 1378 x 1379 x 400 244 /
+// 232, 1000 x 1001 x 513 159 / 167.
+template <int SR, typename T>
 bool chunked_i64(const Problem& p, size_t ws_bytes) {
     if (!std::is_same<T, int64_t>::value || p.M < 32 || p.N < 32) return false;
     const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
     const bool wide = p.M >= 512 && p.N >= 512;
-    const int64_t from = tiles64 <= 256 ? 513 : tiles64 <= 512 ? 193 : !wide ? 161 : tiles64 < 1024 ? 128 : 97;
+    int64_t from = 513;
+    if (SR == tg::SR_MAXMUL && narrow_elements(p)) return false;
+    if (tiles64 > 256 && SR == tg::SR_MAXMUL) from = !wide ? 1501 : tiles64 <= 512 ? 513 : 301;
+    else if (tiles64 > 512 && wide) from = tiles64 < 2048 ? 129 : 97;
+    else if (tiles64 > 256) from = 257;
     if (p.K < from) return false;
     return ws_layout(TG_I64, p.batch, p.M, p.N, p.K, true, 1).total <= ws_bytes &&
            tg::dl64s_fits(p.M, p.N, p.K);
@@ -895,10 +912,10 @@ bool takes_kresg(const Problem& p) {
 // padding for them, on more tiles than CUs (fewer make one round either way).
 // us on MI355X, element loads / generic kernel, whose tiles are 128 x 64:
 //   argmax: f32 500 x (65 x 65 x 97) 126 / 93, x 130 137 / 121, x 200 160 / 176,
-//     1000000 x 2 x 130 784 / 713; i32, whose exact mode is the faster one, 100 x
+//     1000000 x 2 x 130 784 / 713, 53 x (214 x 388 x 115) 81 / 75; i32, whose exact mode is the faster one, 100 x
 //     (100 x 101 x 97) 43 / 38, x 130 47 / 48;
-//   value-only: i32 500 x (65 x 65 x 65) 45 / 36, x 130 69 / 64, x 200 94 / 93,
-//     50000 x 50 x 65 26 / 24, x 130 38 / 40; f32 300000 x 5 x 65 72 / 62, x 200
+//   value-only: i32 500 x (65 x 65 x 65) 45 / 36, x 130 69 / 64, x 200 94 / 93, 1260 x (85 x 31 x 131) 85 / 75,
+//     50000 x 50 x 65 26 / 24, x 130 38 / 40, 100 x 30000 x 97 31 / 27, 2001^2 x 97 33 / 31; f32 300000 x 5 x 65 72 / 62, x 200
 //     146 / 155, 100000 x 33 x 65 29 / 32; four columns or fewer at any K: 1000000
 //     x 2 x 515 1256 / 1121.
 // A few rows are padding in the generic kernel too (3 x 100000 x 97 94 / 129).
@@ -909,9 +926,10 @@ bool elem_padded(const Problem& p, int64_t tiles64, bool i32) {
     if (!argmax && p.N <= 4) return true;
     const double fill = double(p.batch) * double(p.M) * double(p.N) * double(p.K) /
                         (double(tiles64) * 4096 * double((p.K + 31) / 32 * 32));
-    if (argmax) return fill < 0.22 && p.K < 160;
+    if (argmax) return (fill < 0.22 && p.K < 160) || (p.batch > 1 && tiles64 > 1024 && p.K < 128);
     if (p.K < 64) return i32 && fill < 0.3 && p.K < 56;
-    return (p.K < 96 && fill < (i32 ? 0.7 : 0.3)) || (p.K < 200 && fill < 0.22);
+    if (i32 && tiles64 > 448 && p.K < 112 && p.K % 32 != 0) return true;
+    return (p.K < 96 && fill < (i32 ? 0.7 : 0.3)) || (p.K < 200 && fill < (i32 ? 0.3 : 0.22));
 }
 
 // Chooses the kernel.  ws_bytes limits split K (the partials live in the
@@ -987,8 +1005,14 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
         // Aligned problems of up to two tiles per CU whose K the kernels below
         // do not split: its K slices outweigh the element loads (1300^3 f32
         // argmax 134 / 137 us, 4000 x 300 x 2000 180 / 187, 1200 x 1300 x 700
-        // 82 / 89; value-only 94 / 104, 135 / 158, 52 / 58).
-        if (slices > 1 && tiles64 <= 512 && (tiles64 > 256 || p.K % 64 != 0) && take_elem()) return pl;
+        // 82 / 89; value-only 94 / 104, 135 / 158, 52 / 58; the shortest K only for f32
+        // argmax, 1408^2 x 256 43 / 44, i32 51 / 49, value-only x 288 25 / 24).
+        // (i32 argmax of batches neither: 36 x (128 x 320 x 1024) MaxMul 163 / 154).
+        const bool f32_argmax = argmax && std::is_same<T, float>::value;
+        const bool long_enough =
+            tiles64 <= 256 || f32_argmax || (p.K >= 320 && !(argmax && p.batch > 1 && p.K >= 1024));
+        if (slices > 1 && tiles64 <= 512 && (tiles64 > 256 || p.K % 64 != 0) && long_enough && take_elem())
+            return pl;
         if (!exact && !short_tail && !(partial && argmax && p.K <= kExactPartialMaxK)) {
             // Direct-to-LDS kernels (value-only, or argmax beyond the exact
             // range).  Split K when the problem makes too few 64 x 64 tiles
@@ -1079,9 +1103,11 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
         // value-only 1536^2 x 768 200 / 263, 1024^3 111 / 203, 3001^2 x 300
         // 249 / 323.  Short K on few or narrow tiles stays on the generic kernel:
         // argmax (exact mode) 1000^2 x 300 70 / 63, x 384 77 / 78, 1500^2 x 256
-        // 126 / 131, 256 x (64 x 64 x 512) 115 / 103, 8 x 65536 x 512 337 / 331;
-        // value-only 64 x (128 x 128 x 257) 62 / 56, 300 x 5000 x 300 73 / 69, x
-        // 384 84 / 85, 512^2 x 256 35 / 42.
+        // 126 / 131, 1501^2 (element loads) x 256 150 / 140, x 257 142 / 142, 256 x
+        // (64 x 64 x 512) 115 / 103, 128 x (128 x 128 x 449) 183 / 166; value-only 64 x
+        // (128 x 128 x 257) 62 / 56, x 384 67 / 78, 512^2 x 256 35 / 42; in one to two
+        // rounds of tiles 128 x (128 x 128 x 321) 96 / 83, x 513 128 / 127, 64 x 22528 x
+        // 385 93 / 90, x 449 102 / 104, 1224 x 1225 x 300 76 / 71.
         const int64_t tiles = dl64_tiles(p);
         const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
         if (p.K >= 256 && dl64_ws_bytes(p.batch, p.M, p.N, p.K, argmax) <= ws_bytes) {
@@ -1091,9 +1117,13 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
                 return pl;
             }
             const int64_t narrow = p.M < p.N ? p.M : p.N;
-            const bool enough = !argmax ? p.K >= 320 || narrow >= 512
-                                : p.K > exact_tiles_max_k<T>() ||
-                                      (narrow >= 128 && (tiles64 > 512 || p.K > 384));
+            const bool enough =
+                !argmax ? p.K >= 450 || (tiles64 <= 256 || tiles64 > 512 ? p.K >= 320 || narrow >= 512
+                                                                         : p.K >= 350 && narrow >= 512)
+                : p.K > exact_tiles_max_k<T>() ||
+                      (narrow >= 256 &&
+                       (tiles64 <= 512 ? p.K > 384
+                                       : p.K > 256 || tg::dl64s_vectors(p.N, p.K, p.sA, p.sB, p.A, p.B)));
             if (enough && tiles64 >= 64 && tg::dl64s_fits(p.M, p.N, p.K)) {
                 pl.path = argmax ? Path::DL64S : Path::DL64S_VALUE;
                 return pl;
@@ -1102,16 +1132,19 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
     }
     // i64: the chunked and the value-only tiles are tg_gemm_dl64s; the
     // register-staged kernel keeps sizes it does not fit and value-only short K
-    // (us, dl64s / tiles: one round of tiles 1000^2 x 64 15 / 17, x 65 18.7 / 17.8, x
-    // 80 18 / 21; more 1500^2 x 100 53 / 50, x 128 57 / 61, 128 x (128 x 128 x 64)
-    // 26 / 24).
-    const bool i64_dl = std::is_same<T, int64_t>::value && tg::dl64s_fits(p.M, p.N, p.K);
+    // whose last k-tile is mostly padding (us, dl64s / tiles: one round of tiles
+    // 1000^2 x 64 15 / 17, x 65 18.7 / 17.8, x 80 18 / 21, MaxMul x 81 30 / 29; more
+    // 1500^2 x 100 53 / 50, x 128 57 / 61, 3000^2 x 129 183 / 173, x 161 213 / 213,
+    // MaxMul 338 / 319, x 200 384 / 388).
+    const bool i64_dl = std::is_same<T, int64_t>::value && tg::dl64s_fits(p.M, p.N, p.K) &&
+                        !(argmax && SR == tg::SR_MAXMUL && narrow_elements(p));
     const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
     if (!argmax)
-        pl.path = i64_dl && (tiles64 <= 256 ? p.K >= 80 || p.K == 64 : p.K >= 120)
+        pl.path = i64_dl && (tiles64 <= 256 ? p.K >= 96 || (p.K >= 64 && p.K % 16 == 0)
+                                            : p.K >= 192 || p.K == 128)
                       ? Path::DL64S_I64_VALUE
                       : Path::TILES;
-    else if (exact || (p.K <= exact_tiles_max_k<T>() && !chunked_i64<T>(p, ws_bytes)))
+    else if (exact || (p.K <= exact_tiles_max_k<T>() && !chunked_i64<SR, T>(p, ws_bytes)))
         pl.path = Path::TILES_EXACT;
     else
         pl.path = i64_dl ? Path::DL64S_I64 : Path::TILES_CHUNKED;
@@ -1409,14 +1442,14 @@ bool workspace_optional(tg_semiring sr, tg_dtype dt, const Problem& p, const Pla
 // 264, 128 x (128 x 128 x 512) 306 / 190, value-only 1000^2 x 257 63 / 55, 300 x
 // 5000 x 384 104 / 97; i64 argmax 1500^2 x 188 170 / 161, x 300 216 / 245, 1000^3
 // 231 / 267, 256 x (64 x 64 x 1000) 330 / 268.
-bool allocation_pays(tg_dtype dt, const Problem& p, size_t bytes) {
+bool allocation_pays(tg_semiring sr, tg_dtype dt, const Problem& p, size_t bytes) {
     constexpr size_t kMB = size_t(1) << 20;
     const int64_t narrow = p.M < p.N ? p.M : p.N;
     if (p.IDX == nullptr) return p.K >= (narrow >= 512 ? 300 : 400);
     if (bytes <= 2 * kMB) return dt != TG_I32 || p.K >= 128;
     const double products = double(p.batch) * double(p.M) * double(p.N) * double(p.K);
     if (dt == TG_F64) return narrow >= 256 && products >= 8e8;
-    if (dt == TG_I64) return narrow >= 256 && (p.K >= 800 || products >= 5.5e8);
+    if (dt == TG_I64) return narrow >= 256 && (p.K >= 800 || (sr != TG_MAXMUL && products >= 5.5e8));
     return p.K >= (dt == TG_I32 ? 320 : 256) ? bytes <= 64 * kMB || narrow >= 128 : narrow >= 512;
 }
 
@@ -1430,7 +1463,7 @@ size_t own_workspace(tg_semiring sr, tg_dtype dt, const Problem& p, bool* option
     const Plan pl = plan_gemm(sr, dt, p, bytes);
     if (!uses_workspace(pl, argmax)) return 0;
     *optional = workspace_optional(sr, dt, p, pl);
-    return *optional && !allocation_pays(dt, p, bytes) ? 0 : bytes;
+    return *optional && !allocation_pays(sr, dt, p, bytes) ? 0 : bytes;
 }
 
 int gemm_impl(int device, tg_semiring sr, tg_dtype dt, tg_layout layout, const void* A,

@@ -23,6 +23,13 @@ struct Dl64sProblem {
 // slots, one launch).
 bool dl64s_fits(int64_t M, int64_t N, int64_t K);
 
+// 16-byte loads (otherwise element loads): K and N even, 16-byte aligned
+// operands, even batch strides.
+inline bool dl64s_vectors(int64_t N, int64_t K, int64_t sA, int64_t sB, const void* A, const void* B) {
+    auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+    return K % 2 == 0 && N % 2 == 0 && sA % 2 == 0 && sB % 2 == 0 && a16(A) && a16(B);
+}
+
 // K slices per workgroup for `tiles` 64 x 64 tiles.
 int dl64s_slices(int64_t tiles, bool argmax);
 

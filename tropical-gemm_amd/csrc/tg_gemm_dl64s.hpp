@@ -58,12 +58,6 @@ struct Dl64sCfg {
     static_assert(MISC_OFF + 64 <= LDS_BYTES, "epilogue arrays fit the LDS block");
 };
 
-// 16-byte loads (not ELEM): K and N even, 16-byte aligned operands, even batch
-// strides.
-inline bool dl64s_vectors(int64_t N, int64_t K, int64_t sA, int64_t sB, const void* A, const void* B) {
-    auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-    return K % 2 == 0 && N % 2 == 0 && sA % 2 == 0 && sB % 2 == 0 && a16(A) && a16(B);
-}
 // Records of four outputs (record4 with 64-bit compares).
 template <int SR, typename T>
 __device__ __forceinline__ void record4_64(int32_t& c0, int32_t& c1, int32_t& c2, int32_t& c3, T n0,
