@@ -327,6 +327,16 @@ def test_gemm_plan_of_unaligned_short_k_keys():
     ("maxplus", "f32", 1, 16, 16, 65536, True, True), ("maxplus", "f32", 1, 16, 16, 262144, True, False),
     ("maxplus", "f32", 1, 64, 64, (1 << 20) - 1, False, True),  # K that does not split
     ("maxplus", "f64", 1, 64, 64, 1 << 20, True, True),
+    ("maxplus", "f64", 256, 64, 64, 300, True, False), ("maxplus", "f64", 256, 65, 65, 300, True, True),
+    ("maxplus", "f64", 1, 1000, 1000, 300, True, False), ("maxplus", "f64", 1, 700, 700, 300, True, True),
+    ("maxplus", "f64", 1, 300, 5000, 300, False, False), ("maxplus", "f64", 64, 128, 128, 300, False, True),
+    ("maxplus", "f32", 1, 47500, 40, 33, True, False), ("maxplus", "f32", 1, 30000, 40, 33, True, True),
+    ("maxmul", "i32", 1, 100, 15000, 64, True, False), ("maxplus", "f64", 475, 41, 41, 33, True, False),
+    ("maxplus", "f64", 475, 41, 41, 200, True, True), ("maxplus", "f64", 1784, 41, 41, 128, True, False),
+    ("maxplus", "f64", 1, 100, 15000, 64, False, False), ("maxplus", "i64", 1, 15000, 40, 33, True, False),
+    ("maxplus", "i64", 1, 15000, 40, 64, True, True), ("maxmul", "i64", 1220, 64, 64, 161, True, False),
+    ("maxmul", "i64", 1, 100, 50000, 200, True, True), ("maxplus", "i64", 732, 64, 64, 400, False, False),
+    ("maxplus", "i64", 1, 2047, 2049, 1025, False, True), ("maxplus", "i64", 128, 128, 128, 129, False, False),
     ("maxplus", "f32", 256, 48, 48, 512, True, False), ("maxplus", "f32", 64, 48, 48, 512, True, True),
     # Up to 64 columns at short K.
     ("maxplus", "f32", 1, 524288, 64, 2, True, False), ("maxplus", "f32", 1, 524288, 64, 12, True, True),

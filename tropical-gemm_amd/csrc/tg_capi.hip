@@ -1573,6 +1573,53 @@ bool split_outruns_small(const Plan& pl, const Problem& p) {
            double(p.K) * double(tiles64 * 4096) > (argmax ? 4.5e8 : 3.5e8);
 }
 
+// small_output_limit where the other kernel is the generic one or that of the
+// 64-bit 64 x 64 tiles.  The generic tiles' time goes by their number, the few-output
+// kernel's by the outputs, so full tiles and many items draw the line earlier, and
+// K below 64 earliest (its first and last step weigh most).  us on MI355X, small /
+// other:
+//   32-bit: 42 x (452 x 92 x 52) f32 argmax 23 / 28, 2001^2 x 60 45 / 41; 47500 x 40 x
+//     33 f32 argmax 29 / 22, x 64 1.10 times; i32 MaxMul 100 x 11000 x 33 18 / 16, 100 x
+//     15000 x 64 26 / 24;
+//   f64 argmax (the exact mode there has no window loads): 700^3 79 / 111, 1024^3
+//     207 / 149, 256 x (64 x 64 x 300) 93 / 64, 1000^2 x 300 69 / 63, 300 x 5000 x 300
+//     128 / 104, 256 x (65 x 65 x 300) 140 / 216, 475 x (41 x 41 x 33) 24 / 18, x 128 1.07
+//     and x 200 1.00 times, 1784 x (41 x 41 x 128) 186 / 157;
+//   f64 value-only: 700^3 54 / 78, 1024^3 147 / 111, 300 x 5000 x 300 80 / 70, 100 x
+//     16384 x 257 75 / 61; below K = 192 100 x 15000 x 64 25 / 18, 1378 x 1379 x 128
+//     38 / 35, 67 x (128 x 128 x 64) 19 / 17;
+//   i64 argmax: 1536^2 x 768 340 / 365, 2047 x 2049 x 1025 780 / 803, 2048^3 1490 /
+//     1160, in the exact mode's range 2048^2 x 80 83 / 95, 15000 x 40 x 33 17 / 14;
+//     full tiles 1220 x (64 x 64 x 200) 286 / 270; MaxMul 100 x 15000 x 64 1.11 times,
+//     full tiles 1220 x (64 x 64 x 161) 279 / 231, 100 x 50000 x 200 0.90 times;
+//   i64 value-only: 2047 x 2049 x 1025 586 / 652, 3001^2 x 300 388 / 349, 732 x (64 x 64 x
+//     400) 200 / 184, 128 x (128 x 128 x 129) 53 / 47, 463 x (64 x 64 x 64) 25 / 23.
+int64_t small_limit_generic(tg_semiring sr, tg_dtype dt, const Plan& pl, const Problem& p) {
+    constexpr int64_t k1 = int64_t(1) << 10;
+    const bool argmax = p.IDX != nullptr;
+    const int64_t tiles64 = tiles64_of(p);
+    if (dt == TG_F32 || dt == TG_I32) {
+        if (!argmax || p.K >= 96) return 2048 * k1;
+        return dt == TG_F32 ? 1536 * k1 : p.K < 48 ? 1024 * k1 : 1280 * k1;
+    }
+    if (dt == TG_F64) {
+        if (pl.path == Path::TILES_CHUNKED) return 2048 * k1;
+        if (!argmax) return p.K < 192 ? 768 * k1 : tiles64 <= 700 ? 1280 * k1 : 1828 * tiles64;
+        if (p.K < 64 || tiles64 <= 256) return 512 * k1;
+        const int64_t limit = (p.K < 200 ? 1600 : 2048) * tiles64;
+        return limit < 1920 * k1 ? limit : 1920 * k1;
+    }
+    if (!argmax) return p.K < 96 ? 1280 * k1 : p.batch > 1 || p.K < 256 ? 2048 * k1 : 4096 * k1;
+    if (p.K < (sr == TG_MAXMUL ? 64 : 48)) return 512 * k1;
+    const bool full = double(p.batch) * double(p.M) * double(p.N) > 0.9 * 4096 * double(tiles64);
+    if (sr == TG_MAXMUL) {
+        if (p.K < 112) return 1280 * k1;
+        if (full) return 1792 * k1;
+    }
+    if (full && p.batch > 1 && p.K >= 128) return 4096 * k1;
+    return pl.path == Path::TILES_EXACT ? 8192 * k1 : 4096 * k1;
+}
+
 // Outputs (batch x M x N) below which the few-output kernel (tg_gemm_small.hpp)
 // is the faster one, by the path the problem would take otherwise.  Measured
 // on MI355X over 290 shapes of every dtype, with and without argmax (small /
@@ -1591,17 +1638,9 @@ bool split_outruns_small(const Plan& pl, const Problem& p) {
 //     5000 x 48 x 48 7.1 / 9.9, 10000 x 48 x 48 11.9 / 10.2, 5000 x 100 x 100
 //     14 / 17, 10000 x 100 x 100 21 / 18, 5000 x 160 x 160 20.4 / 20.4, 5000 x
 //     256 x 256 43 / 40.
-//   generic tiles, 32-bit (few tiles, or K <= 96): 42 x (452 x 92 x 52) f32
-//     argmax 23 / 28, 2001^2 x 60 45 / 41.
-//   f64: 700^3 argmax 79 / 111, value-only 54 / 78, 1024^3 207 / 149, 147 / 111;
-//     argmax with K < 256 at 100%..130% from half a million outputs (the exact
-//     mode there has no window loads).
-//   i64: argmax 1536^2 x 768 340 / 365, 2047 x 2049 x 1025 780 / 803, 2048^3
-//     1490 / 1160, in the exact mode's range 2048^2 x 80 83 / 95; value-only
-//     2047 x 2049 x 1025 586 / 652, 3001^2 x 300 388 / 349.
 //   K slices in one workgroup on most of the CUs: 256 x (48 x 48 x 512) argmax f32
 //     53 / 46, i32 62 / 52, 64 x (48 x 48 x 512) 21 / 37, 700^2 x 1024 45 / 52.
-int64_t small_output_limit(tg_dtype dt, const Plan& pl, const Problem& p) {
+int64_t small_output_limit(tg_semiring sr, tg_dtype dt, const Plan& pl, const Problem& p) {
     constexpr int64_t k1 = int64_t(1) << 10;
     const bool argmax = p.IDX != nullptr;
     const int64_t narrow = p.M < p.N ? p.M : p.N;
@@ -1640,13 +1679,7 @@ int64_t small_output_limit(tg_dtype dt, const Plan& pl, const Problem& p) {
             if (narrow <= 32) return 2048 * k1;
             return p.K < 256 ? 512 * k1 : pl.splits > 1 && tiles64_of(p) > 160 ? 448 * k1 : 640 * k1;
     }
-    if (dt == TG_I64)
-        return pl.path == Path::TILES_EXACT ? 8192 * k1 : 4096 * k1;
-    if (dt == TG_F64) {
-        if (!argmax || pl.path == Path::TILES_CHUNKED) return 2048 * k1;
-        return p.K < 256 ? 512 * k1 : 1536 * k1;
-    }
-    return 2048 * k1;
+    return small_limit_generic(sr, dt, pl, p);
 }
 
 // What tg_gemm_small runs: `form` is the few-output kernel's launch.
@@ -1664,7 +1697,7 @@ Small choose_small(tg_semiring sr, tg_dtype dt, const Problem& p, tg::SmallForm*
                                 tg::kresg_wave_tiles(p.M, p.N) <= 4096;
     if (few_wave_tiles) pl.path = Path::KRESG;
     // In floating point: batch * M * N of a caller's sizes may pass 2^63.
-    if (double(p.batch) * double(p.M) * double(p.N) < double(small_output_limit(dt, pl, p)) &&
+    if (double(p.batch) * double(p.M) * double(p.N) < double(small_output_limit(sr, dt, pl, p)) &&
         tg::small_form(small_problem(sr, dt, p), form))
         return Small::FEW;
     return few_wave_tiles ? Small::KRESG : Small::NONE;
