@@ -310,6 +310,13 @@ def test_aligned_products_of_two_rounds_of_tiles():
         assert nat.gemm_plan("maxplus", dt, 1408, 1408, k, argmax).startswith(expected)
 
 
+def test_element_load_tiles_of_one_launch():
+    # 2^24 tiles of 256 threads are 2^32, one more than a launch's dimension holds.
+    m = 1 << 30
+    assert nat.gemm_plan("maxplus", "f32", m, 5, 48, False) == "tiles"
+    assert nat.gemm_plan("maxplus", "f32", m - 64, 5, 48, False) == "dl_elem"
+
+
 def test_gemm_plan_of_unaligned_short_k_keys():
     for m, n, k, expected in ((524288, 33, 12, "tiles_exact"), (524288, 33, 20, "kresg"),
                               (65536, 33, 12, "kresg"), (524288, 48, 12, "kresg")):

@@ -988,6 +988,9 @@ Plan plan_typed(const Problem& p, size_t ws_bytes) {
         const int slices = tg::dl_elem_slices(tiles64, p.K, argmax);
         auto take_elem = [&]() {
             if (tiles64 < 64 || !tg::dl_elem_fits<8>(p.M, p.N, p.K)) return false;
+            // One launch holds less than 2^32 threads (256 per tile); the generic
+            // kernel's tiles are twice as high.
+            if (tiles64 / p.batch >= (int64_t(1) << 24)) return false;
             if (tiles64 > 256 && elem_padded(p, tiles64, std::is_same<T, int32_t>::value)) return false;
             if (!argmax) {
                 if (p.K < 48) return false;
